@@ -738,14 +738,18 @@ def main() -> int:
     kern_us = sum(s["solve_kernel_us"] for s in psts)
     visits = sum(s["tile_visits"] for s in psts)
     bpv = sts[0]["bytes_per_visit"]
-    bytes_per_launch = visits * bpv / max(launches, 1)
+    # One launch per step: the resident solve, whose tiles stay in LDS; what it cannot do without
+    # is each cost read once and each time written once.
+    resident = launches == args.steps
+    bytes_per_launch = W * H * 8.0 if resident else visits * bpv / max(launches, 1)
     avg_launch_us = kern_us / max(launches, 1)
     achieved = bytes_per_launch / (avg_launch_us * 1e-6) / 1e9
-    traffic = read_traffic()
+    traffic = None if resident else read_traffic()
     roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5),
             "traffic": None if traffic is None else round(traffic, 1),
-            "kernel": "k_solve_sweep" if kernel == g.KERNEL_SWEEP else "k_solve",
+            "kernel": "k_resident_sweep" if resident else
+                      "k_solve_sweep" if kernel == g.KERNEL_SWEEP else "k_solve",
             "avg_launch_us": round(avg_launch_us, 3),
             "bytes_per_launch": round(bytes_per_launch, 1),
             "launches_per_step": launches / args.steps,

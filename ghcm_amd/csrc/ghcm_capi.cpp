@@ -28,6 +28,7 @@
 #include "ghcm_dev.h"
 #include "ghcm_io.h"
 #include "kernels.h"
+#include "resident.h"
 #include "tile_geom.h"
 
 using namespace ghcm;
@@ -76,6 +77,7 @@ struct ghcm_ctx {
     // device scratch
     DevBuf inst, tinst, qwave, key, mask, tmin, list, ctrl, seeds, jobs, status, tstat, totals, sel;
     DevBuf edge, cedge;         // sweep kernel: edge columns of every tile (time, cost)
+    DevBuf resident;            // resident solve: published borders, states, commands
     DevBuf field_io, time_io;   // staging for the host-buffer entry point
     PinnedBuf io_stage[2];      // pinned parts of host-buffer copies (ping-pong)
     hipEvent_t ev_io[2] = {nullptr, nullptr};
@@ -333,7 +335,7 @@ extern "C" int ghcm_ctx_destroy(ghcm_ctx* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (DevBuf* b : {&ctx->inst, &ctx->tinst, &ctx->qwave, &ctx->key, &ctx->mask, &ctx->tmin,
                       &ctx->list, &ctx->ctrl, &ctx->seeds, &ctx->jobs, &ctx->status,
-                      &ctx->tstat, &ctx->totals, &ctx->sel, &ctx->edge, &ctx->cedge,
+                      &ctx->tstat, &ctx->totals, &ctx->sel, &ctx->edge, &ctx->cedge, &ctx->resident,
                       &ctx->field_io, &ctx->time_io})
         b->release();
     for (PinnedBuf* b : {&ctx->h_ctrl, &ctx->h_seeds, &ctx->h_inst, &ctx->h_jobs,
@@ -639,21 +641,21 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // the whole solve issues no runtime copy.
     HIP_TRY(hipEventRecord(ctx->ev_begin, st));
     // The time fields at +INF and, for the sweep kernels, the tiles' edge columns in one launch.
-    HIP_TRY(launch_solve_init(a, ctx->h_inst.dev_as<GhcmInst>(), n_inst, max_cells, n_sel, d_totals, st,
-                              tw, th, td, kind));
-    if (three_d)
-        HIP_TRY(launch_seed3d(a, ctx->h_seeds.dev_as<uint32_t>(), (uint32_t)n_seeds_total, tw, th, td, st));
-    else
-        HIP_TRY(launch_seed(a, ctx->h_seeds.dev_as<uint32_t>(), (uint32_t)n_seeds_total, tw, th, st));
+    auto enqueue_init = [&]() -> int {
+        HIP_TRY(launch_solve_init(a, ctx->h_inst.dev_as<GhcmInst>(), n_inst, max_cells, n_sel, d_totals, st,
+                                  tw, th, td, kind));
+        if (three_d)
+            HIP_TRY(launch_seed3d(a, ctx->h_seeds.dev_as<uint32_t>(), (uint32_t)n_seeds_total, tw, th, td, st));
+        else
+            HIP_TRY(launch_seed(a, ctx->h_seeds.dev_as<uint32_t>(), (uint32_t)n_seeds_total, tw, th, st));
+        return GHCM_OK;
+    };
 
     uint64_t max_waves = cfg.max_waves ? cfg.max_waves : (uint64_t)8 * T + 100000;
     // Per-tile counters are summed once after the last wave (outside the timed span) and
     // handed over through the progress record; the host polls for this solve's tag.
     bool totals_ready = false;
-    auto publish_totals = [&]() -> int {
-        const uint32_t tag = ++ctx->solve_seq;
-        HIP_TRY(launch_reduce_stats(a.tstat, T, d_totals, st));
-        HIP_TRY(launch_publish_totals(d_totals, a.ctrl, ctx->rec.dev_as<HostRec>(), tag, st));
+    auto await_totals = [&](uint32_t tag) -> int {
         for (uint64_t spins = 0; hr->totals_tag != tag; ++spins) {
             if ((spins & 4095u) == 4095u) {
                 const hipError_t q = hipStreamQuery(st);
@@ -668,9 +670,77 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
         totals_ready = true;
         return GHCM_OK;
     };
+    auto publish_totals = [&]() -> int {
+        const uint32_t tag = ++ctx->solve_seq;
+        HIP_TRY(launch_reduce_stats(a.tstat, T, d_totals, st));
+        HIP_TRY(launch_publish_totals(d_totals, a.ctrl, ctx->rec.dev_as<HostRec>(), tag, st));
+        return await_totals(tag);
+    };
     bool converged = false;
     uint64_t waves_done = 0, visits = 0, inner = 0, improved = 0, kern_launches = 0;
     double kern_us = 0.0;
+
+    // The resident solve (resident.hip): one launch in place of the wave loop, for the 64 x 64
+    // sweep tiles of the default launch mode.  It has no top-n cut, so it takes configurations
+    // whose n fills the chip (at least one tile per CU: the wave loop cuts below that, and a
+    // caller that sets n small asks for the cut) and no wave cap, and grids of up to 32 tiles
+    // per resident work-group (32,768 tiles, 11,500^2 cells on 256 CUs).  Work-groups look at
+    // all their tiles, so its cost per crossing grows with tiles per work-group: 2048^2 (one
+    // tile each) 1,020 -> 540 us, 4096^2 (four) 1,774 -> 1,050 us.
+    const ResidentKernel rk = get_resident_kernel((int)tw, (int)th, kind, cfg.kernel);
+    bool resident_done = false;
+    const uint32_t rgroups = rk.launch ? std::min({(uint32_t)std::max(0, rk.blocks_per_cu()) * (uint32_t)std::max(1, ctx->cus),
+                                                   kResMaxGroups, T})
+                                       : 0u;
+    if (rgroups && !three_d && !host_sched && !noalloc && cfg.launch_mode == 0 && cfg.max_waves == 0 &&
+        n_sel >= (uint32_t)std::max(1, ctx->cus) && (uint64_t)T <= (uint64_t)rgroups * kResMaxOwned) {
+        ResidentArgs ra{};
+        const size_t eb = 1024ull * T, sb = 8ull * kResMaxGroups, cb = 4ull * kResMaxGroups;
+        const size_t total = 2 * eb + 2 * sb + cb + 4ull * kResCtlWords + 12ull * std::max<uint64_t>(1, n_seeds_total);
+        if ((rc = ctx->resident.reserve(total))) return rc;
+        char* const base = ctx->resident.as<char>();
+        ra.inst = d_inst;
+        ra.n_inst = n_inst;
+        ra.tinst = d_tinst;
+        ra.tiles = T;
+        ra.eps = cfg.min_change;
+        ra.edges = reinterpret_cast<uint32_t*>(base);
+        ra.seen = reinterpret_cast<uint32_t*>(base + eb);
+        ra.state = reinterpret_cast<unsigned long long*>(base + 2 * eb);
+        ra.report = reinterpret_cast<unsigned long long*>(base + 2 * eb + sb);
+        ra.cmd = reinterpret_cast<uint32_t*>(base + 2 * eb + 2 * sb);
+        ra.ctl = reinterpret_cast<uint32_t*>(base + 2 * eb + 2 * sb + cb);
+        ra.seeds = ra.ctl + kResCtlWords;
+        ra.n_seeds = (uint32_t)n_seeds_total;
+        ra.rec = ctx->rec.dev_as<HostRec>();
+        ra.tag = ++ctx->solve_seq;
+        HIP_TRY(launch_resident_init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
+        const bool prof = cfg.profile_kernels != 0;
+        while (prof && ctx->ev_prof.size() < 2) {
+            hipEvent_t ev;
+            HIP_TRY(hipEventCreate(&ev));
+            ctx->ev_prof.push_back(ev);
+        }
+        HIP_TRY(rk.launch(ra, rgroups, st, prof ? ctx->ev_prof[0] : nullptr, prof ? ctx->ev_prof[1] : nullptr));
+        HIP_TRY(hipEventRecord(ctx->ev_end, st));
+        if ((rc = await_totals(ra.tag))) return rc;
+        if (prof) {
+            float ms = 0.0f;
+            HIP_TRY(hipEventElapsedTime(&ms, ctx->ev_prof[0], ctx->ev_prof[1]));
+            kern_us = 1000.0 * ms;
+            kern_launches = 1;
+        }
+        if (hr->wave == 0) {
+            resident_done = true;
+            converged = true;
+            waves_done = hr->busy_waves;
+        } else {
+            totals_ready = false;       // given up before it began: the wave loop solves it
+            kern_us = 0.0;
+            kern_launches = 0;
+        }
+    }
+    if (!resident_done && (rc = enqueue_init())) return rc;
 
     // launch_mode 3: tile solve and wave boundary in one launch (sweep kernel).
     const SolveKernel fk = get_fused_kernel((int)tw, (int)th, kind, cfg.kernel);
@@ -683,7 +753,9 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     const bool bsel = cfg.launch_mode == 5;
     const BfKernel bk = get_bf_kernel((int)tw, (int)th, kind, cfg.kernel, wide, bsel);
     const bool bfree = !three_d && !host_sched && (cfg.launch_mode == 4 || bsel) && bk.launch != nullptr;
-    if (bfree) {
+    if (resident_done) {
+        // solved above
+    } else if (bfree) {
         // ---- boundary-free device wave loop ----
         // Each tile launch reads its own list's counts; its first work-group publishes
         // (done << 32) | (wave + 1) into the mapped progress record.  The host keeps `lead`

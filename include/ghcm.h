@@ -95,9 +95,12 @@ typedef struct ghcm_config {
     uint32_t profile_kernels;       /* 1: time every tile-solve launch with HIP events
                                        (fills solve_kernel_us / solve_launches)       */
     uint32_t launch_mode;           /* device scheduler: 0 = one tile-solve launch per
-                                       wave (default), 1 = one persistent cooperative
-                                       launch runs every wave where built (sweep kernel;
-                                       its grid barrier pays agent-scope fences),
+                                       wave (default; 64x64 sweep tiles with n of at least
+                                       one tile per CU and no wave cap are solved by one
+                                       resident launch instead, without waves),
+                                       1 = one persistent cooperative launch runs every
+                                       wave where built (sweep kernel; its grid barrier
+                                       pays agent-scope fences),
                                        2 = chunks of waves replayed as a HIP graph (host
                                        scheduler: each wave's job upload, launch and
                                        status read-back replayed as one graph),
@@ -118,12 +121,15 @@ typedef struct ghcm_config {
 typedef struct ghcm_stats {
     double   duration_total_us;     /* wall time of the solve call                    */
     double   duration_device_us;    /* GPU time between the first and last event      */
-    uint64_t waves;                 /* waves that processed at least one tile         */
-    uint64_t tile_visits;           /* tiles solved (sum over waves)                  */
+    uint64_t waves;                 /* waves that processed at least one tile; resident
+                                       solve: the most sweep rounds of one work-group */
+    uint64_t tile_visits;           /* tiles solved (sum over waves); resident solve:
+                                       sweep rounds over all tiles                    */
     uint64_t tiles_total;           /* tiles in the grid(s)                           */
     uint64_t cells;                 /* W*H summed over instances                      */
     uint64_t inner_iterations;      /* in-tile passes summed over visits              */
-    uint64_t cells_improved;        /* cell commits that lowered a time               */
+    uint64_t cells_improved;        /* cell commits that lowered a time; resident solve:
+                                       finite cells written                           */
     uint32_t converged;             /* 1 if the queue drained                         */
     uint32_t tile_w, tile_h;        /* tile shape used                                */
     uint32_t n_active;              /* n used                                         */

@@ -1,0 +1,128 @@
+"""The resident solve (one launch, tiles kept in LDS, borders exchanged while sweeping) against
+the oracle's FP32 FMM and against the wave loop -- needs an MI355X.
+
+Tolerances: the oracle bar of the parity tests (1e-4 max T, identical INF pattern, fixed-point
+gap within 4 ulp + 2 eps); against the wave loop (launch_mode 4), two fixed points of the same
+FP32 update whose visiting orders differ: 4e-6 max T, about 32 ulp of the largest time.
+"""
+import threading
+
+import numpy as np
+import pytest
+
+import ghcm_amd as g
+import oracle
+from test_gpu_parity import check
+
+pytestmark = pytest.mark.gpu
+CFG = dict(tile_w=64, tile_h=64, kernel=g.KERNEL_SWEEP, n_active=512, inner_iter_cap=1)
+
+
+def _field(rng, h, w, obstacles=0.1):
+    cost = rng.uniform(0.1, 10.0, (h, w)).astype(np.float32)
+    cost[rng.random((h, w)) < obstacles] = np.inf
+    return cost
+
+
+# edges of tiles (63, 64, 65), one row or column, and more tiles than resident work-groups
+# (2100 x 2100 has 1,089 tiles; 70000 x 64 and 64 x 70000 have 1,094)
+@pytest.mark.parametrize("shape", [(1, 1), (1, 200), (200, 1), (63, 64), (64, 65), (65, 63),
+                                   (129, 200), (200, 641), (2100, 2100), (64, 70000), (70000, 64)])
+def test_shapes_obstacles_and_corner_seeds(rng, shape):
+    h, w = shape
+    cost = _field(rng, h, w, 0.1 if min(h, w) > 1 else 0.0)
+    seeds = {(0, 0), (w - 1, h - 1), (min(63, w - 1), min(63, h - 1)), (min(64, w - 1), min(64, h - 1)),
+             (int(rng.integers(0, w)), int(rng.integers(0, h)))}
+    seeds = sorted(seeds)
+    for x, y in seeds:
+        cost[y, x] = 1.0
+    ref = oracle.fmm_f32(cost, seeds)
+    print(f"case resident {shape}", flush=True)
+    with g.Context(0, **CFG) as ctx:
+        for _ in range(2):
+            t, st = ctx.solve(cost, seeds)
+            assert st["converged"] == 1 and st["waves"] > 0
+            check(t, ref, seeds, cost, label=f"resident {shape}")
+        ctx.set_config(launch_mode=4)
+        tw, _ = ctx.solve(cost, seeds)
+    fin = np.isfinite(tw)
+    assert np.array_equal(fin, np.isfinite(t))
+    assert np.max(np.abs(t[fin] - tw[fin])) <= 4e-6 * float(tw[fin].max()) + 1e-6
+
+
+@pytest.mark.parametrize("kind", ["speed_f32", "speed_f16", "speed_bf16"])
+def test_storage_kinds_and_epsilon_zero(kind):
+    speed = g.gen_smooth_speed(333, 270, 9, 12.0, 0.2, 5.0)
+    stored = {"speed_f32": speed.astype(np.float32), "speed_f16": speed.astype(np.float16),
+              "speed_bf16": g.to_bf16(speed)}[kind]
+    back = g.from_bf16(stored) if kind == "speed_bf16" else stored
+    cost = g.cost_from_speed(back)
+    seeds = g.gen_points(333, 270, 10, 5)
+    print(f"case resident {kind}", flush=True)
+    with g.Context(0, min_change=0.0, **CFG) as ctx:
+        t, _ = ctx.solve(stored, seeds, kind=g.KINDS[kind])
+    check(t, oracle.fmm_f32(cost, seeds), seeds, cost, label=kind, eps=0.0)
+
+
+def test_no_seeds_and_walled_off_tiles():
+    cost = np.ones((300, 300), np.float32)
+    with g.Context(0, **CFG) as ctx:
+        t, st = ctx.solve(cost, np.zeros((0, 2), np.uint32))
+        assert np.all(np.isinf(t)) and st["converged"] == 1
+        cost[:, 70] = np.inf
+        t, _ = ctx.solve(cost, [(3, 3)])
+    assert np.all(np.isinf(t[:, 70:]))
+    check(t, oracle.fmm_f32(cost, [(3, 3)]), [(3, 3)], cost)
+
+
+@pytest.mark.parametrize("n_inst", [7, 160])
+def test_uneven_batch(rng, n_inst):
+    """Several instances in one resident launch; 160 of them have more tiles than work-groups."""
+    shapes = [(int(rng.integers(1, 300)), int(rng.integers(1, 300))) for _ in range(n_inst - 1)] + [(300, 1400)]
+    if n_inst > 100:
+        shapes = [(h + 100, w + 100) for h, w in shapes]
+    costs = [_field(rng, h, w, 0.05) for h, w in shapes]
+    seeds = []
+    for c in costs:
+        s = [(int(rng.integers(0, c.shape[1])), int(rng.integers(0, c.shape[0]))) for _ in range(3)]
+        for x, y in s:
+            c[y, x] = 1.0
+        seeds.append(s)
+    print(f"case resident batch {n_inst}", flush=True)
+    with g.Context(0, **dict(CFG, n_active=65536)) as ctx:
+        dev = [(ctx.to_device(c), ctx.alloc(c.shape, np.float32)) for c in costs]
+        st = ctx.solve_batch(g.FIELD_COST_F32, [(d.ptr, t.ptr, c.shape[1], c.shape[0], s)
+                                                for (d, t), c, s in zip(dev, costs, seeds)])
+        assert st["converged"] == 1
+        for (d, t), c, s in zip(dev, costs, seeds):
+            check(t.download(), oracle.fmm_f32(c, s), s, c, label=f"batch {c.shape}")
+            d.free()
+            t.free()
+
+
+def test_contexts_in_threads():
+    """Three contexts solve 2048^2 at once, repeatedly: each wants the whole chip, so launches
+    wait for one another or give way to the wave loop; every result is the same."""
+    speed = g.gen_smooth_speed(2048, 2048, 3, 32.0, 0.1, 10.0)
+    cost = g.cost_from_speed(speed)
+    seeds = g.gen_points(2048, 2048, 4, 3)
+    ref = oracle.fmm_f32(cost, seeds)
+    out, errs = {}, []
+
+    def work(i):
+        try:
+            with g.Context(0, **CFG) as ctx:
+                for _ in range(3):
+                    out[i] = ctx.solve(cost, seeds)[0]
+        except Exception as e:      # noqa: BLE001
+            errs.append(e)
+
+    print("case resident threads", flush=True)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errs, errs
+    for i in range(3):
+        check(out[i], ref, seeds, cost, label=f"thread {i}")
