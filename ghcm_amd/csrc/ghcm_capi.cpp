@@ -683,10 +683,13 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // The resident solve (resident.hip): one launch in place of the wave loop, for the 64 x 64
     // sweep tiles of the default launch mode.  It has no top-n cut, so it takes configurations
     // whose n fills the chip (at least one tile per CU: the wave loop cuts below that, and a
-    // caller that sets n small asks for the cut) and no wave cap, and grids of up to 32 tiles
-    // per resident work-group (32,768 tiles, 11,500^2 cells on 256 CUs).  Work-groups look at
-    // all their tiles, so its cost per crossing grows with tiles per work-group: 2048^2 (one
-    // tile each) 1,020 -> 540 us, 4096^2 (four) 1,774 -> 1,050 us.
+    // caller that sets n small asks for the cut) and no wave cap, and up to 256 tiles per
+    // resident work-group (262,144 tiles on 256 CUs).  2048^2 (one tile each) 1,020 -> 540 us,
+    // 4096^2 (four) 1,774 -> 970 us, a batch of 512 (143) 20.9 -> 13.3 ms.
+    // Up to kScanOwned tiles each, work-groups scan the borders of their closed tiles, above it
+    // they are told: four tiles 1,020 against 1,180 us, eight 1,400 against 1,550, 21 3.76
+    // against 3.38 ms.
+    constexpr uint32_t kScanOwned = 8;
     const ResidentKernel rk = get_resident_kernel((int)tw, (int)th, kind, cfg.kernel);
     bool resident_done = false;
     const uint32_t rgroups = rk.launch ? std::min({(uint32_t)std::max(0, rk.blocks_per_cu()) * (uint32_t)std::max(1, ctx->cus),
@@ -696,25 +699,32 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
         n_sel >= (uint32_t)std::max(1, ctx->cus) && (uint64_t)T <= (uint64_t)rgroups * kResMaxOwned) {
         ResidentArgs ra{};
         const size_t eb = 1024ull * T, sb = 8ull * kResMaxGroups, cb = 4ull * kResMaxGroups;
-        const size_t total = 2 * eb + 2 * sb + cb + 4ull * kResCtlWords + 12ull * std::max<uint64_t>(1, n_seeds_total);
+        const uint32_t want_stride = ((T + rgroups - 1) / rgroups + 15) / 16 * 16;
+        const uint32_t owned = (T + rgroups - 1) / rgroups;
+        const bool scan = owned <= kScanOwned;
+        const size_t wb = scan ? eb : 4ull * kResMaxGroups * want_stride;
+        const size_t tb = sizeof(ResTile) * (size_t)T;
+        const size_t total = eb + wb + tb + 2 * sb + cb + 4ull * kResCtlWords + 16ull * std::max<uint64_t>(1, n_seeds_total);
         if ((rc = ctx->resident.reserve(total))) return rc;
         char* const base = ctx->resident.as<char>();
-        ra.inst = d_inst;
         ra.n_inst = n_inst;
-        ra.tinst = d_tinst;
         ra.tiles = T;
         ra.eps = cfg.min_change;
         ra.edges = reinterpret_cast<uint32_t*>(base);
-        ra.seen = reinterpret_cast<uint32_t*>(base + eb);
-        ra.state = reinterpret_cast<unsigned long long*>(base + 2 * eb);
-        ra.report = reinterpret_cast<unsigned long long*>(base + 2 * eb + sb);
-        ra.cmd = reinterpret_cast<uint32_t*>(base + 2 * eb + 2 * sb);
-        ra.ctl = reinterpret_cast<uint32_t*>(base + 2 * eb + 2 * sb + cb);
+        (scan ? ra.seen : ra.want) = owned > 1 ? reinterpret_cast<uint32_t*>(base + eb) : nullptr;
+        ra.want_stride = want_stride;
+        char* p = base + eb + wb;
+        ra.rtile = reinterpret_cast<ResTile*>(p);
+        ra.state = reinterpret_cast<unsigned long long*>(p += tb);
+        ra.report = reinterpret_cast<unsigned long long*>(p += sb);
+        ra.cmd = reinterpret_cast<uint32_t*>(p += sb);
+        ra.ctl = reinterpret_cast<uint32_t*>(p += cb);
         ra.seeds = ra.ctl + kResCtlWords;
         ra.n_seeds = (uint32_t)n_seeds_total;
         ra.rec = ctx->rec.dev_as<HostRec>();
         ra.tag = ++ctx->solve_seq;
-        HIP_TRY(launch_resident_init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
+        HIP_TRY(launch_resident_init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(),
+                                     rgroups, kind, st));
         const bool prof = cfg.profile_kernels != 0;
         while (prof && ctx->ev_prof.size() < 2) {
             hipEvent_t ev;

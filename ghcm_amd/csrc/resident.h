@@ -20,18 +20,35 @@ enum : uint32_t {
 };
 
 constexpr uint32_t kResMaxGroups = 1024;     // work-groups whose states one of them watches
-constexpr uint32_t kResMaxOwned = 32;        // tiles of one work-group
+constexpr uint32_t kResMaxScan = 32;         // tiles of one work-group that scans their borders
+constexpr uint32_t kResMaxOwned = 256;       // tiles of one work-group (one want a thread)
+
+// What a work-group needs to open a tile: one read.
+struct alignas(16) ResTile {
+    const void* field;       // its first cell in the field and in the times
+    float*      time;
+    uint32_t    w;           // cells per row of the grid
+    uint32_t    ext;         // its columns | rows << 8
+    uint32_t    g;           // its id
+    uint32_t    inst;
+    uint32_t    face[4];     // across side s: id * 4 + side of the border facing it, or kNoTile
+    uint32_t    call[4];     // and where in `want` its owner is told
+    uint32_t    x0, y0;      // its origin
+    uint32_t    pad[2];
+};
 
 struct ResidentArgs {
-    const GhcmInst* inst;
     uint32_t        n_inst;
-    const uint32_t* tinst;   // instance of each tile (null with one instance)
-    const uint32_t* seeds;   // [n_seeds] (x, y, instance)
+    ResTile*        rtile;   // [tiles] by rank (the order in which tiles are dealt out)
+    uint32_t*       seeds;   // [n_seeds] (x, y, instance, rank of its tile)
     uint32_t        n_seeds;
     uint32_t        tiles;
     float           eps;
     uint32_t*       edges;   // [tiles][4][64] published border cells (float bits), side-major
+    // With several tiles to a work-group, one of (the other null):
     uint32_t*       seen;    // [tiles][4][64] the neighbours' facing borders a closed tile was left with
+    uint32_t*       want;    // [groups][want_stride] smallest new border value of an owned tile's neighbours
+    uint32_t        want_stride;
     unsigned long long* state;  // [groups] (acknowledged epoch << 32) | visit counter, odd while busy
     uint32_t*       cmd;     // [groups] epoch to acknowledge, or kCmdDone / kCmdAbort
     uint32_t*       ctl;     // kResCtlWords
@@ -48,6 +65,6 @@ struct ResidentKernel {
 ResidentKernel get_resident_kernel(int tile_w, int tile_h, int kind, int mode);
 // h_inst, h_seeds: device views of the mapped host instance table and source list.
 hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
-                                hipStream_t s);
+                                uint32_t groups, int kind, hipStream_t s);
 
 }  // namespace ghcm

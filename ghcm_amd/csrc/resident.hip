@@ -25,8 +25,12 @@
 //              tile r (in an order that shears the rows, so that a front in any direction meets
 //              many work-groups) belongs to work-group r mod N, which has one of its tiles open
 //              at a time and opens next the one with the smallest new border value.  A closed
-//              tile lives in the time field; seen[] is what its neighbours' borders were.  Only
-//              the owner touches a tile, so its times need no agent-scope access.
+//              tile lives in the time field.  Only the owner touches a tile, so its times need
+//              no agent-scope access.  With few tiles the owner scans the borders that face its
+//              closed tiles against seen[], what they were when it closed them; with many, who
+//              publishes a border then lowers want[] of the tile across, which the owner reads
+//              in one load for all its tiles and withdraws before it reads the borders: what is
+//              announced after that the looks at the then open tile see.
 //   end        a work-group publishes a counter that is odd while it works: odd before its
 //              first border store is issued, even after its last one is visible.  Work-group 0,
 //              when idle, reads all counters; if all are even it sends an epoch, which a
@@ -40,7 +44,8 @@
 //
 // Measured (MI355X, whole calls, wave loop -> this): 256^2 rings 452 -> 231 us, 1531 x 977 smooth
 // 813 -> 339, 2048^2 rings of contrast 1e4 4300 -> 1745, 2048^2 smooth 1020 -> 540, 4096^2
-// smooth 1774 -> 1050, a batch of 48 uneven fields (1,123 tiles) 845 -> 400.
+// smooth 1774 -> 1050, a batch of 48 uneven fields (1,123 tiles) 845 -> 400,
+// a batch of 512 (147 k tiles) 20.9 -> 13.3 ms.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -54,11 +59,18 @@ namespace ghcm {
 
 namespace {
 
+// How a work-group learns that a closed tile of its own has new halo values: it has one tile
+// (never closed), it scans the borders that face them all, or their neighbours' owners tell it.
+enum : int { kOwnOne = 0, kOwnScan = 1, kOwnWant = 2 };
+
 constexpr uint32_t kCmdDone = 0xFFFFFFFFu;
 constexpr uint32_t kCmdAbort = 0xFFFFFFFEu;
 // Sweep steps between two exchanges: 8 against 16 and 32, 4096^2 1,050 against 1,100 and 1,430 us,
 // 2048^2 contrast 1,800 against 1,870 and 2,400 us, smaller grids equal.
 constexpr int kChunk = 8;
+// With many tiles to a work-group all CUs are busy and a front is no longer waited for: a batch of
+// 512 uneven fields 13.3 ms at 16, 13.9 at 8.
+constexpr int kChunkWant = 16;
 // Sweep steps of a round: one ordered pass of all lanes (127) rounded up to the period of the
 // wrapped skew, so that the next round takes up where this one ended.
 constexpr int kSweepRound = 128;
@@ -83,16 +95,6 @@ __device__ __forceinline__ void wait_stores() { __asm__ volatile("s_waitcnt vmcn
 
 __device__ __forceinline__ uint64_t now_ticks() { return __builtin_amdgcn_s_memrealtime(); }
 
-// t improves on t0 by at least eps (strictly): times are compared as bits, so a NaN or a
-// negative value never counts.
-__device__ __forceinline__ bool improves(float t, float t0, float eps) {
-    return __float_as_uint(t) < __float_as_uint(t0) && t0 - t >= eps;
-}
-
-__device__ __forceinline__ float umin_bits(float u, float v) {
-    return __uint_as_float(min(__float_as_uint(u), __float_as_uint(v)));
-}
-
 // OR of `bits` over the four waves; one barrier.  Consecutive calls use different buffers.
 __device__ __forceinline__ uint32_t wg_or(uint32_t bits, uint32_t* buf, int w, int L) {
     if (L == 0) buf[w] = bits;
@@ -100,11 +102,38 @@ __device__ __forceinline__ uint32_t wg_or(uint32_t bits, uint32_t* buf, int w, i
     return buf[0] | buf[1] | buf[2] | buf[3];
 }
 
-// Row y of an instance's tiles is rotated by y times this many tiles before the tiles are dealt
-// out to the work-groups, so that a front along a column of tiles meets as many different
-// work-groups (and XCDs) as one along a row.
-__host__ __device__ __forceinline__ uint32_t resident_shear(uint32_t tiles_x) {
-    return (tiles_x * 3u / 8u) | 1u;
+// The tiles' order: row by row, row ty rotated by ty times shear tiles, so that a front along a
+// column of tiles meets as many different work-groups (and XCDs) as one along a row.
+__device__ __forceinline__ uint32_t shear(uint32_t tiles_x) { return (tiles_x * 3u / 8u) | 1u; }
+__device__ __forceinline__ uint32_t resident_rank(const GhcmInst& in, uint32_t tx, uint32_t ty) {
+    const uint32_t rot = (uint32_t)(((uint64_t)ty * shear(in.tiles_x)) % in.tiles_x);
+    const uint32_t x = tx + rot;
+    return in.tile_base + ty * in.tiles_x + (x >= in.tiles_x ? x - in.tiles_x : x);
+}
+__device__ __forceinline__ void resident_tile(const GhcmInst& in, uint32_t rank, int& tx, int& ty) {
+    const uint32_t lr = rank - in.tile_base, y = lr / in.tiles_x, x = lr - y * in.tiles_x;
+    const uint32_t rot = (uint32_t)(((uint64_t)y * shear(in.tiles_x)) % in.tiles_x);
+    tx = (int)(x >= rot ? x - rot : x + in.tiles_x - rot);
+    ty = (int)y;
+}
+
+// A tile's record as wave-uniform values.
+__device__ __forceinline__ ResTile uniform_tile(const ResTile* p) {
+    static_assert(sizeof(ResTile) % 16 == 0, "whole vectors");
+    ResTile d;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 v[sizeof(ResTile) / 16];
+    uint32_t* const o = reinterpret_cast<uint32_t*>(&d);
+#pragma unroll
+    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) v[i] = gmem(reinterpret_cast<const u32x4*>(p))[i];
+#pragma unroll
+    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) {
+        o[4 * i] = __builtin_amdgcn_readfirstlane(v[i].x);
+        o[4 * i + 1] = __builtin_amdgcn_readfirstlane(v[i].y);
+        o[4 * i + 2] = __builtin_amdgcn_readfirstlane(v[i].z);
+        o[4 * i + 3] = __builtin_amdgcn_readfirstlane(v[i].w);
+    }
+    return d;
 }
 
 // Whether the caller is the last of N to come to the counter at ctl[which]: one counter for the
@@ -117,46 +146,24 @@ __device__ __forceinline__ bool last_in(uint32_t* ctl, uint32_t which, uint32_t 
     return __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == min(N, kResSpread);
 }
 
-// Whether some cell of the LDS tile would still improve from its four neighbours.
-template <int TW, int TH>
-__device__ __forceinline__ bool tile_unsettled(const float* t_s, const float* c_s, int w, int L, float eps) {
-    constexpr int PW = TW + 2, RW = TH / 4;
-    static_assert(TW == 64, "one lane per column");
-    const int r0 = w * RW;
-    const float* const col = t_s + (r0 + 1) * PW + L + 1;
-    const float* const cst = c_s + (r0 + 1) * PW + L + 1;
-    const float* const hal = t_s + (r0 + 1) * PW + (L < 32 ? 0 : PW - 1);
-    float up = col[-PW], mid = col[0];
-    bool res = false;
-#pragma unroll
-    for (int k = 0; k < RW; ++k) {
-        const float down = col[(k + 1) * PW], h = hal[k * PW], c = cst[k * PW];
-        // lanes 0 and 63 have no source lane and keep their halo cell
-        const float l = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(h), __float_as_int(mid), 0x138, 0xF, 0xF, false));
-        const float r = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(h), __float_as_int(mid), 0x130, 0xF, 0xF, false));
-        const float ax = umin_bits(l, r), ay = umin_bits(up, down);
-        res |= improves(godunov_raw(ax, ay, umin_bits(ax, ay), c), mid, eps);
-        up = mid;
-        mid = down;
-    }
-    return res;
-}
-
 }  // namespace
 
-template <int TW, int TH, int KIND>
+template <int TW, int TH, int KIND, int OWN>
 __global__ __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void k_resident_sweep(ResidentArgs a) {
     constexpr int PW = TW + 2, PH = TH + 2, PP = PW * PH, CB = PP + 1;
     constexpr int CPT = TW * TH / kSweepThreads;
+    constexpr int kEvery = OWN == kOwnWant ? kChunkWant : kChunk;
     __shared__ float sh[sweep_lds_words<TW, TH>()];
     __shared__ uint32_t s_or[3][4];
     __shared__ uint32_t s_cmd[2];
     __shared__ uint32_t s_pub;
-    __shared__ uint32_t s_seeded;                      // bit k: owned tile k holds a source
-    __shared__ uint32_t s_key[kResMaxOwned];           // smallest new border value of an owned tile
-    __shared__ uint32_t s_tile[kResMaxOwned];          // its id
-    __shared__ uint32_t s_from[kResMaxOwned][4];       // its neighbours' facing borders (words of a.edges)
+    __shared__ uint32_t s_seeded[kResMaxOwned / 32];   // bit k: owned tile k holds a source
+    __shared__ uint32_t s_opened[kResMaxOwned / 32];   // bit k: owned tile k has been opened
+    __shared__ uint32_t s_best[2][4], s_bk[2][4];      // kOwnWant: each wave's smallest want, and whose it is
+    __shared__ uint32_t s_key[OWN == kOwnScan ? kResMaxScan : 1];       // kOwnScan, of owned tile k: its
+    __shared__ uint32_t s_tile[OWN == kOwnScan ? kResMaxScan : 1];      // neighbours' smallest new border value,
+    __shared__ uint32_t s_from[OWN == kOwnScan ? kResMaxScan : 1][4];   // its id, the borders that face it
     float* const t_s = sh;
     float* const c_s = sh + CB;
     char* const shb = reinterpret_cast<char*>(sh);
@@ -172,26 +179,20 @@ void k_resident_sweep(ResidentArgs a) {
                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         s_pub = 0u;
-        s_seeded = 0u;
     }
+    if (tid < (int)(kResMaxOwned / 32)) s_seeded[tid] = s_opened[tid] = 0u;
     const uint64_t t_start = now_ticks();
 
     // ---- the tiles of this work-group ----
     const uint32_t m = (T - b + N - 1) / N;            // b < N <= T
-    if (tid < (int)m) {
-        const uint32_t r = b + (uint32_t)tid * N;
-        const GhcmInst in = a.inst[a.n_inst == 1 ? 0u : a.tinst[r]];
-        const uint32_t lr = r - in.tile_base, ty = lr / in.tiles_x;
-        const uint32_t rot = (uint32_t)(((uint64_t)ty * resident_shear(in.tiles_x)) % in.tiles_x);
-        uint32_t tx = lr - ty * in.tiles_x;
-        tx = tx >= rot ? tx - rot : tx + in.tiles_x - rot;
-        const uint32_t g = in.tile_base + ty * in.tiles_x + tx;
-        s_tile[tid] = g;
-        for (int s = 0; s < 4; ++s) {
-            const uint32_t nb = tile_neighbour(in.tile_base, in.tiles_x, in.tiles_y, (int)tx, (int)ty, s);
-            s_from[tid][s] = nb == kNoTile ? kNoTile : nb * 256u + (uint32_t)(s ^ 2) * 64u;
+    uint32_t* const want = a.want + (size_t)b * a.want_stride;
+    if constexpr (OWN == kOwnScan) {
+        if (tid < (int)m) {
+            const ResTile& d = a.rtile[b + (uint32_t)tid * N];
+            s_tile[tid] = d.g;
+            for (int q = 0; q < 4; ++q) s_from[tid][q] = d.face[q];
+            s_key[tid] = kInfBits;
         }
-        s_key[tid] = kInfBits;
     }
     // halo ring of the time box (the interior is staged whole)
     for (int i = tid; i < PW; i += kSweepThreads) {
@@ -205,26 +206,26 @@ void k_resident_sweep(ResidentArgs a) {
 
     __syncthreads();
     for (uint32_t i = tid; i < a.n_seeds; i += kSweepThreads) {
-        const uint32_t x = a.seeds[3 * i], y = a.seeds[3 * i + 1];
-        const GhcmInst in = a.inst[a.seeds[3 * i + 2]];
-        const uint32_t g = tile_of_cell(in.tile_base, in.tiles_x, x, y, TW, TH);
-        for (uint32_t k = 0; k < m; ++k)
-            if (s_tile[k] == g) {
-                s_key[k] = 0u;
-                atomicOr(&s_seeded, 1u << k);
-            }
+        const uint32_t r = a.seeds[4 * i + 3];
+        if (r % N == b) {
+            const uint32_t k = r / N;
+            atomicOr(&s_seeded[k >> 5], 1u << (k & 31u));
+            if constexpr (OWN == kOwnScan) s_key[k] = 0u;
+            if constexpr (OWN == kOwnWant) st_agent(&want[k], 0u);
+        }
     }
+    wait_stores();
     __syncthreads();
 
     // ---- the open tile: in LDS, wave w keeping its side w ----
-    uint32_t cur = kNoTile, cg = 0u, rounds = 0u, reached = 0u, opened = 0u;
-    const uint32_t seeded = __builtin_amdgcn_readfirstlane(s_seeded);
+    uint32_t cur = kNoTile, cg = 0u, rounds = 0u, reached = 0u;
     int sx = 0, sy = 0, W = 0;
     char* tb = nullptr;
     bool act = false;
     int q_own = PW + 1, q_halo = 0;
     const uint32_t* from = a.edges;
     uint32_t* to = a.edges;
+    uint32_t* call = nullptr;           // the want of the tile across this side
     float halo = __builtin_inff();      // the neighbour's border cell, as last read
     float sent = __builtin_inff();      // this tile's border cell, as last published
 
@@ -240,76 +241,83 @@ void k_resident_sweep(ResidentArgs a) {
             }
         }
     };
-    // Read owned tile k into LDS; its halo and its published borders go to registers.
+    // Read owned tile k, write the open one back meanwhile, and put k in its place.
     auto open = [&](uint32_t k) {
-        cur = k;
-        cg = __builtin_amdgcn_readfirstlane(s_tile[k]);
-        const uint32_t ii = a.n_inst == 1 ? 0u : __builtin_amdgcn_readfirstlane(a.tinst[cg]);
-        const GhcmInst in = uniform_inst(a.inst[ii]);
+        const ResTile d = uniform_tile(a.rtile + (b + k * N));
         // A tile opened for the first time is +INF but for its sources: nothing is read.
-        const bool fresh = ((opened >> k) & 1u) == 0u;
-        opened |= 1u << k;
-        int tx, ty;
-        tile_xy(cg - in.tile_base, in.tiles_x, tx, ty);
-        const int ox = tx * TW, oy = ty * TH;
-        W = (int)in.w;
-        sx = tile_extent(W, ox, TW);
-        sy = tile_extent((int)in.h, oy, TH);
-        tb = reinterpret_cast<char*>(in.time) + ((int64_t)oy * W + ox) * 4;
-        const char* const fb = static_cast<const char*>(in.field) + ((int64_t)oy * W + ox) * (int64_t)field_bytes<KIND>();
-        const int len = (w & 1) ? sx : sy;
-        const uint32_t fo = __builtin_amdgcn_readfirstlane(s_from[k][w]);
-        act = fo != kNoTile && L < len;
-        from = a.edges + (fo == kNoTile ? 0u : fo) + L;
-        to = a.edges + (size_t)cg * 256 + (size_t)w * 64 + L;
+        const bool fresh = ((s_opened[k >> 5] >> (k & 31u)) & 1u) == 0u;
+        const int nsx = (int)(d.ext & 0xFFu), nsy = (int)(d.ext >> 8);
+        const char* const fb = static_cast<const char*>(d.field);
+        char* const nt = reinterpret_cast<char*>(d.time);
+        const int c = tid % TW, r0 = tid / TW;
+        const int len = (w & 1) ? nsx : nsy;
+        const uint32_t face = w == 0 ? d.face[0] : w == 1 ? d.face[1] : w == 2 ? d.face[2] : d.face[3];
+        const uint32_t told = w == 0 ? d.call[0] : w == 1 ? d.call[1] : w == 2 ? d.call[2] : d.call[3];
+        const bool nact = face != kNoTile && L < len;
+        const uint32_t* const nfrom = a.edges + (size_t)(face == kNoTile ? 0u : face) * 64 + L;
+        uint32_t* const nto = a.edges + ((size_t)d.g * 4 + w) * 64 + L;
+        // Cells past the grid read the tile's first cell and become +INF (no load waits on a branch).
+        float tv[CPT], cv[CPT];
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+            const int r = r0 + (kSweepThreads / TW) * j;
+            const uint32_t off = c < nsx && r < nsy ? (uint32_t)r * d.w + (uint32_t)c : 0u;
+            cv[j] = load_cost_at<KIND>(fb + off * field_bytes<KIND>());
+            tv[j] = __builtin_inff();
+        }
+        if (!fresh) {
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) {
+                const int r = r0 + (kSweepThreads / TW) * j;
+                const uint32_t off = c < nsx && r < nsy ? (uint32_t)r * d.w + (uint32_t)c : 0u;
+                tv[j] = *gmem(reinterpret_cast<const float*>(nt + off * 4u));
+            }
+        }
+        const float nhalo = nact ? __uint_as_float(ld_agent(nfrom)) : __builtin_inff();
+        const float nsent = nact ? __uint_as_float(ld_agent(nto)) : __builtin_inff();
+        if (cur != kNoTile) {
+            commit();
+            if constexpr (OWN == kOwnScan) a.seen[(size_t)cg * 256 + w * 64 + L] = __float_as_uint(halo);
+            __syncthreads();
+        }
+        cur = k;
+        cg = d.g;
+        sx = nsx;
+        sy = nsy;
+        W = (int)d.w;
+        tb = nt;
+        act = nact;
+        from = nfrom;
+        to = nto;
+        if constexpr (OWN == kOwnWant) call = a.want + told;
+        halo = nhalo;
+        sent = nsent;
         // box words of lane L's border cell and of the halo cell across this side
         const int Lc = min(L, len - 1);
         q_own = w == 0 ? (Lc + 1) * PW + 1 : w == 2 ? (Lc + 1) * PW + sx : w == 1 ? PW + Lc + 1 : sy * PW + Lc + 1;
         q_halo = w == 0 ? q_own - 1 : w == 2 ? q_own + 1 : w == 1 ? q_own - PW : q_own + PW;
-        halo = act ? __uint_as_float(ld_agent(from)) : __builtin_inff();
-        sent = act ? __uint_as_float(ld_agent(to)) : __builtin_inff();
-        // Cells past the grid read the tile's first cell and become +INF (no load waits on a branch).
-        constexpr int kBatch = CPT / 2;
-#pragma unroll 1
-        for (int k0 = 0; k0 < CPT; k0 += kBatch) {
-            float tv[kBatch], cv[kBatch];
-            const int c = tid % TW, r0 = tid / TW + (kSweepThreads / TW) * k0;
 #pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                const int r = r0 + (kSweepThreads / TW) * j;
-                const uint32_t off = c < sx && r < sy ? (uint32_t)r * (uint32_t)W + (uint32_t)c : 0u;
-                cv[j] = load_cost_at<KIND>(fb + off * field_bytes<KIND>());
-                tv[j] = __builtin_inff();
-            }
-            if (!fresh) {
-#pragma unroll
-                for (int j = 0; j < kBatch; ++j) {
-                    const int r = r0 + (kSweepThreads / TW) * j;
-                    const uint32_t off = c < sx && r < sy ? (uint32_t)r * (uint32_t)W + (uint32_t)c : 0u;
-                    tv[j] = *gmem(reinterpret_cast<const float*>(tb + off * 4u));
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                const int r = r0 + (kSweepThreads / TW) * j;
-                const bool in_grid = c < sx && r < sy;
-                t_s[(r + 1) * PW + c + 1] = in_grid ? tv[j] : __builtin_inff();
-                c_s[(r + 1) * PW + c + 1] = in_grid ? cv[j] : __builtin_inff();
-            }
+        for (int j = 0; j < CPT; ++j) {
+            const int r = r0 + (kSweepThreads / TW) * j;
+            const bool in_grid = c < sx && r < sy;
+            t_s[(r + 1) * PW + c + 1] = in_grid ? tv[j] : __builtin_inff();
+            c_s[(r + 1) * PW + c + 1] = in_grid ? cv[j] : __builtin_inff();
         }
         // A partial tile's last column or row has no neighbour; its far halo stays +INF.
         if (act) t_s[q_halo] = halo;
         else if (L < ((w & 1) ? TW : TH))
             t_s[w == 0 ? (L + 1) * PW : w == 2 ? (L + 1) * PW + PW - 1 : w == 1 ? L + 1 : (PH - 1) * PW + L + 1] = __builtin_inff();
-        if (fresh && ((seeded >> k) & 1u)) {
-            __syncthreads();
+        const bool sources = fresh && ((s_seeded[k >> 5] >> (k & 31u)) & 1u);
+        __syncthreads();
+        if (fresh && tid == 0) s_opened[k >> 5] |= 1u << (k & 31u);
+        if (sources) {
             for (uint32_t i = tid; i < a.n_seeds; i += kSweepThreads) {
-                const int x = (int)a.seeds[3 * i] - ox, y = (int)a.seeds[3 * i + 1] - oy;
-                if (a.seeds[3 * i + 2] == ii && x >= 0 && x < sx && y >= 0 && y < sy) t_s[(y + 1) * PW + x + 1] = 0.0f;
+                const int x = (int)(a.seeds[4 * i] - d.x0), y = (int)(a.seeds[4 * i + 1] - d.y0);
+                if (a.seeds[4 * i + 2] == d.inst && x >= 0 && x < sx && y >= 0 && y < sy) t_s[(y + 1) * PW + x + 1] = 0.0f;
             }
         }
     };
-    if (m == 1u) open(0u);
+    if (OWN == kOwnOne || m == 1u) open(0u);
 
     // ---- every work-group is running, or none goes on ----
     if (tid == 0) {
@@ -350,7 +358,7 @@ void k_resident_sweep(ResidentArgs a) {
     for (uint32_t k = 0; k < kResMaxGroups / kSweepThreads; ++k) ver[k] = 0u;
     uint32_t poll = 0;
     // The open tile has cells that would improve.
-    bool work = m == 1u && seeded != 0u;
+    bool work = (OWN == kOwnOne || m == 1u) && (s_seeded[0] & 1u);
     while (go) {
         if (work) {
             if (!(st & 1u)) {
@@ -361,17 +369,35 @@ void k_resident_sweep(ResidentArgs a) {
             float ahead = __builtin_inff();        // the neighbour's border cell, being loaded
             if (act) ahead = __uint_as_float(ld_agent(from));
             bool ch = false;
+            // With several tiles to a work-group the neighbour's owner is told as well, once the
+            // border is visible (at the next exchange): key is the smallest value not yet told.
+            uint32_t key = kInfBits;
+            auto tell = [&]() {
+                if (OWN == kOwnWant && key != kInfBits) {
+                    if (L == 0) __hip_atomic_fetch_min(call, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    key = kInfBits;
+                }
+            };
             auto publish = [&]() {
                 const float mine = t_s[q_own];
-                if (act && __float_as_uint(mine) < __float_as_uint(sent) && __float_as_uint(mine) < __float_as_uint(halo)) {
+                const bool out = act && __float_as_uint(mine) < __float_as_uint(sent) && __float_as_uint(mine) < __float_as_uint(halo);
+                if (out) {
                     st_agent(to, __float_as_uint(mine));
                     sent = mine;
                 }
+                if (OWN == kOwnWant && __ballot(out))
+                    key = min(key, __float_as_uint(wave_min(out ? mine : __builtin_inff())));
             };
             auto exchange = [&]() {
-                if (__float_as_uint(ahead) < __float_as_uint(halo)) {
-                    halo = ahead;
-                    t_s[q_halo] = ahead;
+                const float v = ahead;
+                if constexpr (OWN == kOwnWant) {
+                    // The load of `ahead` was issued after the last border store: both are done.
+                    __asm__ volatile("" ::"v"(v) : "memory");
+                    tell();
+                }
+                if (__float_as_uint(v) < __float_as_uint(halo)) {
+                    halo = v;
+                    t_s[q_halo] = v;
                     ch = true;
                 }
                 if (!pub) {
@@ -390,11 +416,13 @@ void k_resident_sweep(ResidentArgs a) {
             // box is checked cell by cell.
             do {
                 ch = false;
+                // The open tile's neighbours announce what the exchanges see by themselves.
+                if (OWN == kOwnWant && tid == 0) st_agent(&want[cur], kInfBits);
                 switch (w) {
-                    case 0: sweep_round<TW, TH, 1, true, kChunk, kSweepRound>(shb, L, exchange); break;
-                    case 1: sweep_round<TW, TH, -1, true, kChunk, kSweepRound>(shb, L, exchange); break;
-                    case 2: sweep_round<TW, TH, 1, false, kChunk, kSweepRound>(shb, L, exchange); break;
-                    default: sweep_round<TW, TH, -1, false, kChunk, kSweepRound>(shb, L, exchange); break;
+                    case 0: sweep_round<TW, TH, 1, true, kEvery, kSweepRound>(shb, L, exchange); break;
+                    case 1: sweep_round<TW, TH, -1, true, kEvery, kSweepRound>(shb, L, exchange); break;
+                    case 2: sweep_round<TW, TH, 1, false, kEvery, kSweepRound>(shb, L, exchange); break;
+                    default: sweep_round<TW, TH, -1, false, kEvery, kSweepRound>(shb, L, exchange); break;
                 }
                 ++rounds;
                 const bool stop = (rounds & 1023u) == 0u && ld_agent(&a.cmd[b]) == kCmdAbort;
@@ -416,6 +444,10 @@ void k_resident_sweep(ResidentArgs a) {
                     more = (r & 4u) == 0u;
                 }
             } while (more);
+            if (OWN == kOwnWant && key != kInfBits) {
+                wait_stores();
+                tell();
+            }
             work = false;
         }
         // ---- look at every owned tile's neighbours ----
@@ -442,8 +474,9 @@ void k_resident_sweep(ResidentArgs a) {
                 }
                 bits = (__ballot(busy) ? 4u : 0u) | (__ballot(differs) ? 8u : 0u) | (__ballot(unacked) ? 16u : 0u);
             }
-            if (m > 1u) {
-                // four tiles' loads at a time
+            bool asked = false;                 // kOwnWant: the open tile's own want is set
+            if (OWN == kOwnScan && m > 1u) {
+                // the neighbours' borders of every closed tile, four tiles' loads at a time
                 for (uint32_t k0 = 0; k0 < m; k0 += 4) {
                     float nv[4], sv[4];
 #pragma unroll
@@ -453,7 +486,7 @@ void k_resident_sweep(ResidentArgs a) {
                         nv[j] = sv[j] = __builtin_inff();
                         // (cells past a partial tile's extent are never published and stay +INF)
                         if (k0 + j < m && k != cur && fo != kNoTile) {
-                            nv[j] = __uint_as_float(ld_agent(a.edges + fo + L));
+                            nv[j] = __uint_as_float(ld_agent(a.edges + (size_t)fo * 64 + L));
                             sv[j] = __uint_as_float(a.seen[(size_t)__builtin_amdgcn_readfirstlane(s_tile[k]) * 256 + w * 64 + L]);
                         }
                     }
@@ -468,13 +501,29 @@ void k_resident_sweep(ResidentArgs a) {
                     }
                 }
             }
+            if (OWN == kOwnWant && m > 1u) {
+                uint32_t own = (uint32_t)tid < m ? ld_agent(&want[tid]) : kInfBits;
+                asked = (uint32_t)tid == cur && own != kInfBits;
+                if (asked) {
+                    // The borders it announces are visible and the next look reads them.
+                    st_agent(&want[tid], kInfBits);
+                    wait_stores();
+                    own = kInfBits;
+                }
+                const float best = wave_min(__uint_as_float(own));
+                const unsigned long long who = __ballot(own == __float_as_uint(best));
+                if (L == 0) {
+                    s_best[poll & 1u][w] = __float_as_uint(best);
+                    s_bk[poll & 1u][w] = (uint32_t)(w * 64 + __builtin_ctzll(who));
+                }
+            }
             const bool ch = __float_as_uint(v) < __float_as_uint(halo);
             if (ch) {
                 halo = v;
                 t_s[q_halo] = v;
             }
             if (tid == 0) s_cmd[poll & 1u] = c;
-            const uint32_t r = any4(bits | (__ballot(ch) ? 2u : 0u));
+            const uint32_t r = any4(bits | (__ballot(ch) ? 2u : 0u) | (__ballot(asked) ? 32u : 0u));
             cmd = s_cmd[poll & 1u];
             if (cmd == kCmdDone || cmd == kCmdAbort) break;
             if (r & 2u) {
@@ -484,29 +533,39 @@ void k_resident_sweep(ResidentArgs a) {
                 }
                 continue;
             }
-            if (m > 1u) {
-                // the owned tile with the smallest new value, if any has one
+            if (r & 32u) continue;
+            if (OWN != kOwnOne && m > 1u) {
+                // the owned tile with the smallest new border value, if any has one
                 uint32_t best = kInfBits, bk = 0u;
-                for (uint32_t k = 0; k < m; ++k) {
-                    const uint32_t key = s_key[k];
-                    if (key < best) { best = key; bk = k; }
+                if constexpr (OWN == kOwnScan) {
+                    for (uint32_t k = 0; k < m; ++k) {
+                        const uint32_t v2 = s_key[k];
+                        if (v2 < best) { best = v2; bk = k; }
+                    }
+                    __syncthreads();        // every wave has read the keys
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t v2 = s_best[poll & 1u][i];
+                        if (v2 < best) { best = v2; bk = s_bk[poll & 1u][i]; }
+                    }
                 }
                 best = __builtin_amdgcn_readfirstlane(best);
                 bk = __builtin_amdgcn_readfirstlane(bk);
-                __syncthreads();        // every wave has read the keys
                 if (best != kInfBits) {
-                    if (tid == 0) s_key[bk] = kInfBits;
+                    // Each wave withdraws the want before it reads its side's border (open() waits
+                    // for the tile's record first): what is announced later is seen by the looks
+                    // at the open tile.
+                    if constexpr (OWN == kOwnScan) {
+                        if (tid == 0) s_key[bk] = kInfBits;
+                    } else {
+                        if (L == 0) st_agent(&want[bk], kInfBits);
+                    }
                     // The visit counter turns odd before anything of the new tile is published.
                     if (!(st & 1u)) {
                         ++st;
                         if (tid == 0) st_agent64(&a.state[b], ((unsigned long long)acked << 32) | st);
                     }
-                    if (cur != kNoTile) {
-                        commit();
-                        a.seen[(size_t)cg * 256 + w * 64 + L] = __float_as_uint(halo);
-                    }
-                    wait_stores();
-                    __syncthreads();
                     open(bk);
                     __syncthreads();
                     idle = false;
@@ -566,15 +625,12 @@ void k_resident_sweep(ResidentArgs a) {
         if (cur != kNoTile) commit();
         // Tiles that no front reached.
         for (uint32_t k = 0; k < m; ++k) {
-            if ((opened >> k) & 1u) continue;
-            const uint32_t g = s_tile[k];
-            const GhcmInst in = uniform_inst(a.inst[a.n_inst == 1 ? 0u : a.tinst[g]]);
-            int tx, ty;
-            tile_xy(g - in.tile_base, in.tiles_x, tx, ty);
-            const int ox = tx * TW, oy = ty * TH;
+            if ((s_opened[k >> 5] >> (k & 31u)) & 1u) continue;
+            const ResTile d = uniform_tile(a.rtile + (b + k * N));
+            const int ex = (int)(d.ext & 0xFFu), ey = (int)(d.ext >> 8);
             for (int i = tid; i < TW * TH; i += kSweepThreads) {
-                const int x = ox + i % TW, y = oy + i / TW;
-                if (x < (int)in.w && y < (int)in.h) gmem(in.time)[(size_t)y * in.w + x] = __builtin_inff();
+                const int x = i % TW, y = i / TW;
+                if (x < ex && y < ey) gmem(d.time)[(size_t)y * d.w + x] = __builtin_inff();
             }
         }
     }
@@ -619,49 +675,100 @@ void k_resident_sweep(ResidentArgs a) {
     }
 }
 
-// The state of a resident solve, in one launch: instance table, tile map and sources copied
-// from mapped host memory, borders at +INF, every work-group counted as busy.
-__global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const uint32_t* h_seeds) {
+// The state of a resident solve, in one launch: the tiles' records and the sources (with the
+// rank of their tile) from the mapped host tables, borders at +INF, every work-group busy.
+template <int TW, int TH, int FB>
+__global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const uint32_t* h_seeds, uint32_t N) {
     const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     const uint4 inf4 = make_uint4(kInfBits, kInfBits, kInfBits, kInfBits);
     uint4* const e4 = reinterpret_cast<uint4*>(a.edges);
     uint4* const s4 = reinterpret_cast<uint4*>(a.seen);
     for (size_t i = i0; i < (size_t)a.tiles * 64; i += stride) {
         e4[i] = inf4;
-        s4[i] = inf4;
+        if (a.seen) s4[i] = inf4;
     }
+    if (a.want)
+        for (size_t i = i0; i < (size_t)kResMaxGroups * a.want_stride; i += stride) a.want[i] = kInfBits;
     for (size_t i = i0; i < kResMaxGroups; i += stride) {
         a.state[i] = 1ull;
         a.cmd[i] = 0u;
     }
     for (size_t i = i0; i < kResCtlWords; i += stride) a.ctl[i] = 0u;
-    for (size_t i = i0; i < 3ull * a.n_seeds; i += stride) const_cast<uint32_t*>(a.seeds)[i] = h_seeds[i];
-    for (uint32_t j = blockIdx.x; j < a.n_inst; j += gridDim.x) {
+    for (size_t i = i0; i < a.n_seeds; i += stride) {
+        const uint32_t x = h_seeds[3 * i], y = h_seeds[3 * i + 1], j = h_seeds[3 * i + 2];
         const GhcmInst in = h_inst[j];
-        if (threadIdx.x == 0) const_cast<GhcmInst*>(a.inst)[j] = in;
-        if (a.tinst)
-            for (uint32_t t = threadIdx.x; t < inst_tiles(in); t += blockDim.x)
-                const_cast<uint32_t*>(a.tinst)[in.tile_base + t] = j;
+        a.seeds[4 * i] = x;
+        a.seeds[4 * i + 1] = y;
+        a.seeds[4 * i + 2] = j;
+        a.seeds[4 * i + 3] = resident_rank(in, x / TW, y / TH);
+    }
+    // Tile records: with few instances several blocks share one.
+    const uint32_t share = gridDim.x > a.n_inst ? gridDim.x / a.n_inst : 1u;
+    for (uint32_t j = blockIdx.x / share; j < a.n_inst; j += gridDim.x / share) {
+        if (blockIdx.x / share >= gridDim.x / share) break;
+        const GhcmInst in = h_inst[j];
+        const uint32_t nt = in.tiles_x * in.tiles_y;
+        for (uint32_t t = (blockIdx.x % share) * blockDim.x + threadIdx.x; t < nt; t += share * blockDim.x) {
+            int tx, ty;
+            resident_tile(in, in.tile_base + t, tx, ty);
+            ResTile d;
+            d.g = in.tile_base + (uint32_t)ty * in.tiles_x + (uint32_t)tx;
+            d.inst = j;
+            d.w = in.w;
+            d.x0 = (uint32_t)tx * TW;
+            d.y0 = (uint32_t)ty * TH;
+            const size_t org = (size_t)d.y0 * in.w + d.x0;
+            d.field = static_cast<const char*>(in.field) + org * FB;
+            d.time = in.time + org;
+            d.ext = (uint32_t)tile_extent((int)in.w, (int)d.x0, TW) | (uint32_t)tile_extent((int)in.h, (int)d.y0, TH) << 8;
+            for (int s = 0; s < 4; ++s) {
+                const uint32_t nb = tile_neighbour(in.tile_base, in.tiles_x, in.tiles_y, tx, ty, s);
+                d.face[s] = nb == kNoTile ? kNoTile : nb * 4u + (uint32_t)(s ^ 2);
+                const uint32_t r = nb == kNoTile ? 0u : resident_rank(in, (uint32_t)(tx + side_dx(s)), (uint32_t)(ty + side_dy(s)));
+                d.call[s] = (r % N) * a.want_stride + r / N;
+            }
+            d.pad[0] = d.pad[1] = 0u;
+            a.rtile[in.tile_base + t] = d;
+        }
     }
 }
 
-template <int TW, int TH, int KIND>
-static hipError_t launch_resident_t(const ResidentArgs& a, uint32_t groups, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
-    if (groups == 0 || groups > a.tiles || groups > kResMaxGroups || a.tiles > groups * kResMaxOwned)
-        return hipErrorInvalidValue;
+template <int TW, int TH, int KIND, int OWN>
+static hipError_t launch_own(const ResidentArgs& a, uint32_t groups, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     if (ev0 && ev1)
-        hipExtLaunchKernelGGL((k_resident_sweep<TW, TH, KIND>), dim3(groups), dim3(kSweepThreads), 0, s, ev0, ev1, 0, a);
+        hipExtLaunchKernelGGL((k_resident_sweep<TW, TH, KIND, OWN>), dim3(groups), dim3(kSweepThreads), 0, s, ev0, ev1, 0, a);
     else
-        hipLaunchKernelGGL((k_resident_sweep<TW, TH, KIND>), dim3(groups), dim3(kSweepThreads), 0, s, a);
+        hipLaunchKernelGGL((k_resident_sweep<TW, TH, KIND, OWN>), dim3(groups), dim3(kSweepThreads), 0, s, a);
     return hipGetLastError();
 }
 
 template <int TW, int TH, int KIND>
+static hipError_t launch_resident_t(const ResidentArgs& a, uint32_t groups, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+    if (groups == 0 || groups > a.tiles || groups > kResMaxGroups || (uint64_t)a.tiles > (uint64_t)groups * kResMaxOwned)
+        return hipErrorInvalidValue;
+    if (a.tiles == groups) return launch_own<TW, TH, KIND, kOwnOne>(a, groups, s, ev0, ev1);
+    if (a.seen) {
+        if (a.tiles > groups * kResMaxScan) return hipErrorInvalidValue;
+        return launch_own<TW, TH, KIND, kOwnScan>(a, groups, s, ev0, ev1);
+    }
+    if (!a.want || (uint64_t)groups * a.want_stride < a.tiles) return hipErrorInvalidValue;
+    return launch_own<TW, TH, KIND, kOwnWant>(a, groups, s, ev0, ev1);
+}
+
+template <int TW, int TH, int KIND>
 static int occ_resident_t() {
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_resident_sweep<TW, TH, KIND>, kSweepThreads, 0) != hipSuccess)
-        return 0;
-    return nb;
+    int least = 0;
+    auto with = [&](auto kernel) {
+        int nb = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kSweepThreads, 0) != hipSuccess) nb = 0;
+        least = nb;
+    };
+    with(k_resident_sweep<TW, TH, KIND, kOwnOne>);
+    int n = least;
+    with(k_resident_sweep<TW, TH, KIND, kOwnScan>);
+    n = least < n ? least : n;
+    with(k_resident_sweep<TW, TH, KIND, kOwnWant>);
+    return least < n ? least : n;
 }
 
 ResidentKernel get_resident_kernel(int tw, int th, int kind, int mode) {
@@ -676,9 +783,12 @@ ResidentKernel get_resident_kernel(int tw, int th, int kind, int mode) {
 }
 
 hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
-                                hipStream_t s) {
-    const uint32_t blocks = a.tiles < 1024u ? a.tiles : 1024u;
-    hipLaunchKernelGGL(k_resident_init, dim3(blocks), dim3(256), 0, s, a, h_inst, h_seeds);
+                                uint32_t groups, int kind, hipStream_t s) {
+    const dim3 grid(a.tiles < 1024u ? a.tiles : 1024u), block(256);
+    if (kind <= 1)
+        hipLaunchKernelGGL((k_resident_init<64, 64, 4>), grid, block, 0, s, a, h_inst, h_seeds, groups);
+    else
+        hipLaunchKernelGGL((k_resident_init<64, 64, 2>), grid, block, 0, s, a, h_inst, h_seeds, groups);
     return hipGetLastError();
 }
 

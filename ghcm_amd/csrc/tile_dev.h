@@ -278,4 +278,43 @@ __device__ __forceinline__ void sweep_round(char* const shb, const int L, F betw
     }
 }
 
+// t improves on t0 by at least eps (strictly): times are compared as bits, so a NaN or a
+// negative value never counts.
+__device__ __forceinline__ bool improves(float t, float t0, float eps) {
+    return __float_as_uint(t) < __float_as_uint(t0) && t0 - t >= eps;
+}
+
+__device__ __forceinline__ float umin_bits(float u, float v) {
+    return __uint_as_float(min(__float_as_uint(u), __float_as_uint(v)));
+}
+
+// Whether a cell of this lane's part of the LDS tile would improve from its four neighbours by at
+// least eps; on no lane of the four waves: the tile is settled with respect to its halo.  Wave w
+// checks a quarter of the rows, lane L column L; the rows roll through registers and the left and
+// right neighbours come by DPP, so a cell costs three LDS reads (its lower neighbour, its cost and
+// the halo cell for the outer lanes).
+template <int TW, int TH>
+__device__ __forceinline__ bool tile_unsettled(const float* t_s, const float* c_s, int w, int L, float eps) {
+    constexpr int PW = TW + 2, RW = TH / 4;
+    static_assert(TW == 64, "one lane per column");
+    const int r0 = w * RW;
+    const float* const col = t_s + (r0 + 1) * PW + L + 1;
+    const float* const cst = c_s + (r0 + 1) * PW + L + 1;
+    const float* const hal = t_s + (r0 + 1) * PW + (L < 32 ? 0 : PW - 1);
+    float up = col[-PW], mid = col[0];
+    bool res = false;
+#pragma unroll
+    for (int k = 0; k < RW; ++k) {
+        const float down = col[(k + 1) * PW], h = hal[k * PW], c = cst[k * PW];
+        // lanes 0 and 63 have no source lane and keep their halo cell
+        const float l = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(h), __float_as_int(mid), 0x138, 0xF, 0xF, false));
+        const float r = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(h), __float_as_int(mid), 0x130, 0xF, 0xF, false));
+        const float ax = umin_bits(l, r), ay = umin_bits(up, down);
+        res |= improves(godunov_raw(ax, ay, umin_bits(ax, ay), c), mid, eps);
+        up = mid;
+        mid = down;
+    }
+    return res;
+}
+
 }  // namespace ghcm
