@@ -690,64 +690,84 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // they are told: four tiles 1,020 against 1,180 us, eight 1,400 against 1,550, 21 3.76
     // against 3.38 ms.
     constexpr uint32_t kScanOwned = 8;
-    const ResidentKernel rk = get_resident_kernel((int)tw, (int)th, kind, cfg.kernel);
+    // The one-wave tiles (resident_wave.hip) likewise, one wave64 per tile with the tile in
+    // registers, up to the resident waves (8,184 tiles of 8x8 or 6,136 of 16x16 on 256 CUs; larger
+    // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
+    // 16x16 FIM tiles 3,837 -> 455 us.
     bool resident_done = false;
-    const uint32_t rgroups = rk.launch ? std::min({(uint32_t)std::max(0, rk.blocks_per_cu()) * (uint32_t)std::max(1, ctx->cus),
-                                                   kResMaxGroups, T})
-                                       : 0u;
-    if (rgroups && !three_d && !host_sched && !noalloc && cfg.launch_mode == 0 && cfg.max_waves == 0 &&
-        n_sel >= (uint32_t)std::max(1, ctx->cus) && (uint64_t)T <= (uint64_t)rgroups * kResMaxOwned) {
-        ResidentArgs ra{};
-        const size_t eb = 1024ull * T, sb = 8ull * kResMaxGroups, cb = 4ull * kResMaxGroups;
-        const uint32_t want_stride = ((T + rgroups - 1) / rgroups + 15) / 16 * 16;
-        const uint32_t owned = (T + rgroups - 1) / rgroups;
-        const bool scan = owned <= kScanOwned;
-        const size_t wb = scan ? eb : 4ull * kResMaxGroups * want_stride;
-        const size_t tb = sizeof(ResTile) * (size_t)T;
-        const size_t total = eb + wb + tb + 2 * sb + cb + 4ull * kResCtlWords + 16ull * std::max<uint64_t>(1, n_seeds_total);
-        if ((rc = ctx->resident.reserve(total))) return rc;
-        char* const base = ctx->resident.as<char>();
-        ra.n_inst = n_inst;
-        ra.tiles = T;
-        ra.eps = cfg.min_change;
-        ra.edges = reinterpret_cast<uint32_t*>(base);
-        (scan ? ra.seen : ra.want) = owned > 1 ? reinterpret_cast<uint32_t*>(base + eb) : nullptr;
-        ra.want_stride = want_stride;
-        char* p = base + eb + wb;
-        ra.rtile = reinterpret_cast<ResTile*>(p);
-        ra.state = reinterpret_cast<unsigned long long*>(p += tb);
-        ra.report = reinterpret_cast<unsigned long long*>(p += sb);
-        ra.cmd = reinterpret_cast<uint32_t*>(p += sb);
-        ra.ctl = reinterpret_cast<uint32_t*>(p += cb);
-        ra.seeds = ra.ctl + kResCtlWords;
-        ra.n_seeds = (uint32_t)n_seeds_total;
-        ra.rec = ctx->rec.dev_as<HostRec>();
-        ra.tag = ++ctx->solve_seq;
-        HIP_TRY(launch_resident_init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(),
-                                     rgroups, kind, st));
-        const bool prof = cfg.profile_kernels != 0;
-        while (prof && ctx->ev_prof.size() < 2) {
-            hipEvent_t ev;
-            HIP_TRY(hipEventCreate(&ev));
-            ctx->ev_prof.push_back(ev);
-        }
-        HIP_TRY(rk.launch(ra, rgroups, st, prof ? ctx->ev_prof[0] : nullptr, prof ? ctx->ev_prof[1] : nullptr));
-        HIP_TRY(hipEventRecord(ctx->ev_end, st));
-        if ((rc = await_totals(ra.tag))) return rc;
-        if (prof) {
-            float ms = 0.0f;
-            HIP_TRY(hipEventElapsedTime(&ms, ctx->ev_prof[0], ctx->ev_prof[1]));
-            kern_us = 1000.0 * ms;
-            kern_launches = 1;
-        }
-        if (hr->wave == 0) {
-            resident_done = true;
-            converged = true;
-            waves_done = hr->busy_waves;
-        } else {
-            totals_ready = false;       // given up before it began: the wave loop solves it
-            kern_us = 0.0;
-            kern_launches = 0;
+    const uint32_t cus = (uint32_t)std::max(1, ctx->cus);
+    if (!three_d && !host_sched && !noalloc && cfg.launch_mode == 0 && cfg.max_waves == 0 && n_sel >= cus) {
+        const ResidentKernel rk = get_resident_kernel((int)tw, (int)th, kind, cfg.kernel);
+        const ResidentWaveKernel wk = get_resident_wave_kernel((int)tw, (int)th, kind, cfg.kernel);
+        const uint64_t fit = (uint64_t)std::max(0, rk.launch ? rk.blocks_per_cu() : wk.launch ? wk.blocks_per_cu() : 0) * cus;
+        // Work-groups: for the sweep tiles as many as fit, each with a share of the tiles; for the
+        // one-wave tiles one per eight tiles (and one more that watches).
+        const uint32_t groups = rk.launch ? (uint32_t)std::min<uint64_t>({fit, kResMaxGroups, T}) : (T + 7u) / 8u;
+        const bool fits = rk.launch ? groups && (uint64_t)T <= (uint64_t)groups * kResMaxOwned
+                                    : wk.launch && T <= kResMaxWaveTiles && groups + 1u <= fit;
+        if (fits) {
+            const uint32_t owned = rk.launch ? (T + groups - 1) / groups : 1u;
+            const bool scan = owned <= kScanOwned;
+            const uint32_t states = rk.launch ? kResMaxGroups : kResMaxWaveTiles;
+            ResidentArgs ra{};
+            ra.n_inst = n_inst;
+            ra.tiles = T;
+            ra.eps = cfg.min_change;
+            ra.want_stride = (owned + 15u) / 16u * 16u;
+            ra.n_seeds = (uint32_t)n_seeds_total;
+            ra.rec = ctx->rec.dev_as<HostRec>();
+            // One buffer: its parts in turn, each on a 256-byte boundary.
+            const size_t eb = rk.launch ? 1024ull * T : 4ull * wk.inbox_words * T;
+            size_t need = 0;
+            auto part = [&need](size_t bytes) {
+                const size_t at = need;
+                need += (bytes + 255) & ~size_t(255);
+                return at;
+            };
+            const size_t o_edges = part(eb), o_seen = part(owned > 1 && scan ? eb : 0),
+                         o_want = part(owned > 1 && !scan ? 4ull * kResMaxGroups * ra.want_stride : 0),
+                         o_tile = part(sizeof(ResTile) * (size_t)T), o_state = part(8ull * states),
+                         o_report = part(8ull * states), o_cmd = part(4ull * states), o_ctl = part(4ull * kResCtlWords),
+                         o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
+            if ((rc = ctx->resident.reserve(need))) return rc;
+            char* const base = ctx->resident.as<char>();
+            ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
+            if (owned > 1 && scan) ra.seen = reinterpret_cast<uint32_t*>(base + o_seen);
+            if (owned > 1 && !scan) ra.want = reinterpret_cast<uint32_t*>(base + o_want);
+            ra.rtile = reinterpret_cast<ResTile*>(base + o_tile);
+            ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
+            ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
+            ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
+            ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
+            ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
+            ra.tag = ++ctx->solve_seq;
+            const bool prof = cfg.profile_kernels != 0;
+            while (prof && ctx->ev_prof.size() < 2) {
+                hipEvent_t ev;
+                HIP_TRY(hipEventCreate(&ev));
+                ctx->ev_prof.push_back(ev);
+            }
+            const hipEvent_t e0 = prof ? ctx->ev_prof[0] : nullptr, e1 = prof ? ctx->ev_prof[1] : nullptr;
+            const GhcmInst* const inst_view = ctx->h_inst.dev_as<GhcmInst>();
+            const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
+            HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, seeds_view, groups, kind, st)
+                              : wk.init(ra, inst_view, seeds_view, kind, st));
+            HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
+            HIP_TRY(hipEventRecord(ctx->ev_end, st));
+            if ((rc = await_totals(ra.tag))) return rc;
+            if (hr->wave == 0) {
+                resident_done = true;
+                converged = true;
+                waves_done = hr->busy_waves;
+                if (prof) {
+                    float ms = 0.0f;
+                    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+                    kern_us = 1000.0 * ms;
+                    kern_launches = 1;
+                }
+            } else {
+                totals_ready = false;       // given up before it began: the wave loop solves it
+            }
         }
     }
     if (!resident_done && (rc = enqueue_init())) return rc;

@@ -67,4 +67,17 @@ ResidentKernel get_resident_kernel(int tile_w, int tile_h, int kind, int mode);
 hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
                                 uint32_t groups, int kind, hipStream_t s);
 
+// The one-wave tiles (8x8, 16x16, 32x8, 32x32): one wave64 per tile, the tile in its registers.
+// Here `edges` holds the tiles' inboxes (`inbox_words` each: the cells across each border, written
+// by the neighbours), and state, cmd and report are per tile.
+constexpr uint32_t kResMaxWaveTiles = 8192;
+struct ResidentWaveKernel {
+    hipError_t (*launch)(const ResidentArgs&, uint32_t groups, hipStream_t, hipEvent_t ev0, hipEvent_t ev1);
+    hipError_t (*init)(const ResidentArgs&, const GhcmInst* h_inst, const uint32_t* h_seeds, int kind, hipStream_t);
+    int (*blocks_per_cu)();
+    uint32_t inbox_words;
+};
+// mode: 0 systolic, 1 FIM.
+ResidentWaveKernel get_resident_wave_kernel(int tile_w, int tile_h, int kind, int mode);
+
 }  // namespace ghcm

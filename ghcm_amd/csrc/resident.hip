@@ -52,6 +52,7 @@
 
 #include "ghcm_dev.h"
 #include "resident.h"
+#include "resident_dev.h"
 #include "tile_dev.h"
 #include "tile_geom.h"
 
@@ -63,8 +64,6 @@ namespace {
 // (never closed), it scans the borders that face them all, or their neighbours' owners tell it.
 enum : int { kOwnOne = 0, kOwnScan = 1, kOwnWant = 2 };
 
-constexpr uint32_t kCmdDone = 0xFFFFFFFFu;
-constexpr uint32_t kCmdAbort = 0xFFFFFFFEu;
 // Sweep steps between two exchanges: 8 against 16 and 32, 4096^2 1,050 against 1,100 and 1,430 us,
 // 2048^2 contrast 1,800 against 1,870 and 2,400 us, smaller grids equal.
 constexpr int kChunk = 8;
@@ -74,76 +73,11 @@ constexpr int kChunkWant = 16;
 // Sweep steps of a round: one ordered pass of all lanes (127) rounded up to the period of the
 // wrapped skew, so that the next round takes up where this one ended.
 constexpr int kSweepRound = 128;
-constexpr uint64_t kJoinTicks = 20000;               // 200 us of the 100 MHz counter
-constexpr uint64_t kLimitTicks = 2000000000ull;      // 20 s
-
-__device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long ld_agent64(const unsigned long long* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent64(unsigned long long* p, unsigned long long v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Every vector memory operation of this wave so far is complete (stores: visible at the scope
-// they were made).
-__device__ __forceinline__ void wait_stores() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-__device__ __forceinline__ uint64_t now_ticks() { return __builtin_amdgcn_s_memrealtime(); }
-
 // OR of `bits` over the four waves; one barrier.  Consecutive calls use different buffers.
 __device__ __forceinline__ uint32_t wg_or(uint32_t bits, uint32_t* buf, int w, int L) {
     if (L == 0) buf[w] = bits;
     __syncthreads();
     return buf[0] | buf[1] | buf[2] | buf[3];
-}
-
-// The tiles' order: row by row, row ty rotated by ty times shear tiles, so that a front along a
-// column of tiles meets as many different work-groups (and XCDs) as one along a row.
-__device__ __forceinline__ uint32_t shear(uint32_t tiles_x) { return (tiles_x * 3u / 8u) | 1u; }
-__device__ __forceinline__ uint32_t resident_rank(const GhcmInst& in, uint32_t tx, uint32_t ty) {
-    const uint32_t rot = (uint32_t)(((uint64_t)ty * shear(in.tiles_x)) % in.tiles_x);
-    const uint32_t x = tx + rot;
-    return in.tile_base + ty * in.tiles_x + (x >= in.tiles_x ? x - in.tiles_x : x);
-}
-__device__ __forceinline__ void resident_tile(const GhcmInst& in, uint32_t rank, int& tx, int& ty) {
-    const uint32_t lr = rank - in.tile_base, y = lr / in.tiles_x, x = lr - y * in.tiles_x;
-    const uint32_t rot = (uint32_t)(((uint64_t)y * shear(in.tiles_x)) % in.tiles_x);
-    tx = (int)(x >= rot ? x - rot : x + in.tiles_x - rot);
-    ty = (int)y;
-}
-
-// A tile's record as wave-uniform values.
-__device__ __forceinline__ ResTile uniform_tile(const ResTile* p) {
-    static_assert(sizeof(ResTile) % 16 == 0, "whole vectors");
-    ResTile d;
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 v[sizeof(ResTile) / 16];
-    uint32_t* const o = reinterpret_cast<uint32_t*>(&d);
-#pragma unroll
-    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) v[i] = gmem(reinterpret_cast<const u32x4*>(p))[i];
-#pragma unroll
-    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) {
-        o[4 * i] = __builtin_amdgcn_readfirstlane(v[i].x);
-        o[4 * i + 1] = __builtin_amdgcn_readfirstlane(v[i].y);
-        o[4 * i + 2] = __builtin_amdgcn_readfirstlane(v[i].z);
-        o[4 * i + 3] = __builtin_amdgcn_readfirstlane(v[i].w);
-    }
-    return d;
-}
-
-// Whether the caller is the last of N to come to the counter at ctl[which]: one counter for the
-// work-groups b with equal b % kResSpread, and one for the last of each, each on its own line.
-__device__ __forceinline__ bool last_in(uint32_t* ctl, uint32_t which, uint32_t b, uint32_t N) {
-    const uint32_t j = b % kResSpread, members = (N - j + kResSpread - 1u) / kResSpread;
-    uint32_t* const c = ctl + which;
-    if (__hip_atomic_fetch_add(c + (1u + j) * kCounterStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != members)
-        return false;
-    return __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == min(N, kResSpread);
 }
 
 }  // namespace
@@ -173,11 +107,7 @@ void k_resident_sweep(ResidentArgs a) {
     const float eps = a.eps;
 
     if (tid == 0) {
-        if (last_in(a.ctl, kResArrived, b, N)) {
-            uint32_t expect = 0u;
-            __hip_atomic_compare_exchange_strong(&a.ctl[kResDecision], &expect, 1u, __ATOMIC_RELAXED,
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        if (last_in(a.ctl, kResArrived, b, N)) decide(a.ctl, 1u);
         s_pub = 0u;
     }
     if (tid < (int)(kResMaxOwned / 32)) s_seeded[tid] = s_opened[tid] = 0u;
@@ -320,19 +250,7 @@ void k_resident_sweep(ResidentArgs a) {
     if (OWN == kOwnOne || m == 1u) open(0u);
 
     // ---- every work-group is running, or none goes on ----
-    if (tid == 0) {
-        uint32_t d;
-        while ((d = ld_agent(&a.ctl[kResDecision])) == 0u) {
-            if (now_ticks() - t_start > kJoinTicks) {
-                uint32_t expect = 0u;
-                if (__hip_atomic_compare_exchange_strong(&a.ctl[kResDecision], &expect, 2u, __ATOMIC_RELAXED,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    st_agent(&a.ctl[kResFailed], 1u);
-            }
-            __builtin_amdgcn_s_sleep(4);
-        }
-        s_cmd[0] = d;
-    }
+    if (tid == 0) s_cmd[0] = await_decision(a.ctl, t_start);
     __syncthreads();
     const bool go = s_cmd[0] != 2u;
     __syncthreads();
@@ -665,71 +583,7 @@ void k_resident_sweep(ResidentArgs a) {
             sum_cells += red[kSweepThreads + i];
             most = max(most, (uint32_t)red[2 * kSweepThreads + i]);
         }
-        sys_store64(&a.rec->totals[0], sum_rounds);
-        sys_store64(&a.rec->totals[1], sum_rounds);
-        sys_store64(&a.rec->totals[2], sum_cells);
-        sys_store(&a.rec->wave, ld_agent(&a.ctl[kResFailed]));
-        sys_store(&a.rec->busy_waves, most);
-        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        sys_store(&a.rec->totals_tag, a.tag);
-    }
-}
-
-// The state of a resident solve, in one launch: the tiles' records and the sources (with the
-// rank of their tile) from the mapped host tables, borders at +INF, every work-group busy.
-template <int TW, int TH, int FB>
-__global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const uint32_t* h_seeds, uint32_t N) {
-    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
-    const uint4 inf4 = make_uint4(kInfBits, kInfBits, kInfBits, kInfBits);
-    uint4* const e4 = reinterpret_cast<uint4*>(a.edges);
-    uint4* const s4 = reinterpret_cast<uint4*>(a.seen);
-    for (size_t i = i0; i < (size_t)a.tiles * 64; i += stride) {
-        e4[i] = inf4;
-        if (a.seen) s4[i] = inf4;
-    }
-    if (a.want)
-        for (size_t i = i0; i < (size_t)kResMaxGroups * a.want_stride; i += stride) a.want[i] = kInfBits;
-    for (size_t i = i0; i < kResMaxGroups; i += stride) {
-        a.state[i] = 1ull;
-        a.cmd[i] = 0u;
-    }
-    for (size_t i = i0; i < kResCtlWords; i += stride) a.ctl[i] = 0u;
-    for (size_t i = i0; i < a.n_seeds; i += stride) {
-        const uint32_t x = h_seeds[3 * i], y = h_seeds[3 * i + 1], j = h_seeds[3 * i + 2];
-        const GhcmInst in = h_inst[j];
-        a.seeds[4 * i] = x;
-        a.seeds[4 * i + 1] = y;
-        a.seeds[4 * i + 2] = j;
-        a.seeds[4 * i + 3] = resident_rank(in, x / TW, y / TH);
-    }
-    // Tile records: with few instances several blocks share one.
-    const uint32_t share = gridDim.x > a.n_inst ? gridDim.x / a.n_inst : 1u;
-    for (uint32_t j = blockIdx.x / share; j < a.n_inst; j += gridDim.x / share) {
-        if (blockIdx.x / share >= gridDim.x / share) break;
-        const GhcmInst in = h_inst[j];
-        const uint32_t nt = in.tiles_x * in.tiles_y;
-        for (uint32_t t = (blockIdx.x % share) * blockDim.x + threadIdx.x; t < nt; t += share * blockDim.x) {
-            int tx, ty;
-            resident_tile(in, in.tile_base + t, tx, ty);
-            ResTile d;
-            d.g = in.tile_base + (uint32_t)ty * in.tiles_x + (uint32_t)tx;
-            d.inst = j;
-            d.w = in.w;
-            d.x0 = (uint32_t)tx * TW;
-            d.y0 = (uint32_t)ty * TH;
-            const size_t org = (size_t)d.y0 * in.w + d.x0;
-            d.field = static_cast<const char*>(in.field) + org * FB;
-            d.time = in.time + org;
-            d.ext = (uint32_t)tile_extent((int)in.w, (int)d.x0, TW) | (uint32_t)tile_extent((int)in.h, (int)d.y0, TH) << 8;
-            for (int s = 0; s < 4; ++s) {
-                const uint32_t nb = tile_neighbour(in.tile_base, in.tiles_x, in.tiles_y, tx, ty, s);
-                d.face[s] = nb == kNoTile ? kNoTile : nb * 4u + (uint32_t)(s ^ 2);
-                const uint32_t r = nb == kNoTile ? 0u : resident_rank(in, (uint32_t)(tx + side_dx(s)), (uint32_t)(ty + side_dy(s)));
-                d.call[s] = (r % N) * a.want_stride + r / N;
-            }
-            d.pad[0] = d.pad[1] = 0u;
-            a.rtile[in.tile_base + t] = d;
-        }
+        report_totals(a, sum_rounds, sum_rounds, sum_cells, most);
     }
 }
 
@@ -784,12 +638,7 @@ ResidentKernel get_resident_kernel(int tw, int th, int kind, int mode) {
 
 hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
                                 uint32_t groups, int kind, hipStream_t s) {
-    const dim3 grid(a.tiles < 1024u ? a.tiles : 1024u), block(256);
-    if (kind <= 1)
-        hipLaunchKernelGGL((k_resident_init<64, 64, 4>), grid, block, 0, s, a, h_inst, h_seeds, groups);
-    else
-        hipLaunchKernelGGL((k_resident_init<64, 64, 2>), grid, block, 0, s, a, h_inst, h_seeds, groups);
-    return hipGetLastError();
+    return launch_init<64, 64>(a, h_inst, h_seeds, groups, 256u, kResMaxGroups, kind, s);
 }
 
 }  // namespace ghcm

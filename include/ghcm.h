@@ -95,8 +95,9 @@ typedef struct ghcm_config {
     uint32_t profile_kernels;       /* 1: time every tile-solve launch with HIP events
                                        (fills solve_kernel_us / solve_launches)       */
     uint32_t launch_mode;           /* device scheduler: 0 = one tile-solve launch per
-                                       wave (default; 64x64 sweep tiles with n of at least
-                                       one tile per CU and no wave cap are solved by one
+                                       wave (default; 64x64 sweep tiles, and grids of up to
+                                       8,184 systolic or FIM tiles, with n of at least one
+                                       tile per CU and no wave cap are solved by one
                                        resident launch instead, without waves),
                                        1 = one persistent cooperative launch runs every
                                        wave where built (sweep kernel; its grid barrier
@@ -122,9 +123,9 @@ typedef struct ghcm_stats {
     double   duration_total_us;     /* wall time of the solve call                    */
     double   duration_device_us;    /* GPU time between the first and last event      */
     uint64_t waves;                 /* waves that processed at least one tile; resident
-                                       solve: the most sweep rounds of one work-group */
+                                       solve: the most rounds of one work-group       */
     uint64_t tile_visits;           /* tiles solved (sum over waves); resident solve:
-                                       sweep rounds over all tiles                    */
+                                       rounds of sweeps or passes over all tiles      */
     uint64_t tiles_total;           /* tiles in the grid(s)                           */
     uint64_t cells;                 /* W*H summed over instances                      */
     uint64_t inner_iterations;      /* in-tile passes summed over visits              */

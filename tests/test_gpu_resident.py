@@ -64,6 +64,49 @@ def test_storage_kinds_and_epsilon_zero(kind):
     check(t, oracle.fmm_f32(cost, seeds), seeds, cost, label=kind, eps=0.0)
 
 
+WAVE_TILES = [(g.KERNEL_SYSTOLIC, (8, 8)), (g.KERNEL_FIM, (8, 8)), (g.KERNEL_SYSTOLIC, (16, 16)),
+              (g.KERNEL_FIM, (16, 16)), (g.KERNEL_SYSTOLIC, (32, 8)), (g.KERNEL_SYSTOLIC, (32, 32))]
+
+
+# one cell, edges of tiles, and for 8x8 tiles the most that fit (8,184) and more (wave loop)
+@pytest.mark.parametrize("kernel,tile", WAVE_TILES)
+@pytest.mark.parametrize("shape", [(1, 1), (1, 130), (7, 9), (8, 33), (17, 64), (129, 200), (720, 720), (744, 704), (744, 712)])
+def test_one_wave_tiles(rng, kernel, tile, shape):
+    h, w = shape
+    cost = _field(rng, h, w, 0.1 if min(h, w) > 1 else 0.0)
+    seeds = sorted({(0, 0), (w - 1, h - 1), (min(7, w - 1), min(7, h - 1)), (min(8, w - 1), min(8, h - 1)),
+                    (int(rng.integers(0, w)), int(rng.integers(0, h)))})
+    for x, y in seeds:
+        cost[y, x] = 1.0
+    ref = oracle.fmm_f32(cost, seeds)
+    print(f"case resident kernel={kernel} tile={tile} {shape}", flush=True)
+    with g.Context(0, tile_w=tile[0], tile_h=tile[1], kernel=kernel) as ctx:
+        for _ in range(2):
+            t, st = ctx.solve(cost, seeds)
+            assert st["converged"] == 1 and st["waves"] > 0
+            check(t, ref, seeds, cost, label=f"{kernel} {tile} {shape}")
+
+
+@pytest.mark.parametrize("kind", ["speed_f32", "speed_f16", "speed_bf16"])
+def test_one_wave_tiles_storage_and_batch(rng, kind):
+    """Several instances, stored as speed, at eps = 0; hundreds of sources in one of them."""
+    speeds = [g.gen_smooth_speed(w, h, 3 + w, 8.0, 0.2, 5.0) for w, h in ((100, 90), (33, 150), (8, 8))]
+    stored = [{"speed_f32": s.astype(np.float32), "speed_f16": s.astype(np.float16),
+               "speed_bf16": g.to_bf16(s) if kind == "speed_bf16" else None}[kind] for s in speeds]
+    costs = [g.cost_from_speed(g.from_bf16(s) if kind == "speed_bf16" else s) for s in stored]
+    seeds = [[(5, 5), (99, 89)], g.gen_points(33, 150, 4, 300), [(3, 4)]]
+    print(f"case resident one-wave {kind}", flush=True)
+    with g.Context(0, min_change=0.0) as ctx:
+        dev = [(ctx.to_device(s), ctx.alloc(s.shape, np.float32)) for s in stored]
+        st = ctx.solve_batch(g.KINDS[kind], [(d.ptr, t.ptr, s.shape[1], s.shape[0], q)
+                                             for (d, t), s, q in zip(dev, stored, seeds)])
+        assert st["converged"] == 1
+        for (d, t), c, q in zip(dev, costs, seeds):
+            check(t.download(), oracle.fmm_f32(c, q), q, c, label=f"{kind} {c.shape}", eps=0.0)
+            d.free()
+            t.free()
+
+
 def test_no_seeds_and_walled_off_tiles():
     cost = np.ones((300, 300), np.float32)
     with g.Context(0, **CFG) as ctx:
