@@ -13,7 +13,7 @@ namespace ghcm {
 constexpr uint32_t kResSpread = 32;          // arrival counters beside the top one
 enum : uint32_t {
     kResDecision = 0,    // 0: undecided, 1: every work-group is running, 2: not all came in time
-    kResFailed = 1,      // 1: given up (declined, or out of time); the wave loop takes over
+    kResFailed = 1,      // 1: given up for want of time; the wave loop takes over
     kResArrived = kCounterStride,                                   // work-groups running
     kResLeft = kResArrived + (1 + kResSpread) * kCounterStride,     // work-groups done
     kResCtlWords = kResLeft + (1 + kResSpread) * kCounterStride
@@ -79,5 +79,40 @@ struct ResidentWaveKernel {
 };
 // mode: 0 systolic, 1 FIM.
 ResidentWaveKernel get_resident_wave_kernel(int tile_w, int tile_h, int kind, int mode);
+
+// 3-D sweep tiles (64 x 8 x 8), one work-group per tile.  `edges` holds kRes3Words a tile (34 rows of
+// 64 border cells), `seeds` (x, y, z, rank of its tile).
+constexpr uint32_t kRes3Words = 34 * 64;
+struct alignas(16) ResTile3 {
+    const void* field;       // its first cell in the field and in the times
+    float*      time;
+    uint64_t    plane;       // cells per plane of the grid
+    uint32_t    w;           // cells per row
+    uint32_t    ext;         // its columns | rows << 8 | planes << 16
+    uint32_t    g;           // its id
+    uint32_t    x0, y0, z0;
+    uint32_t    face[6];     // the tile across side s (0 x-, 1 y-, 2 x+, 3 y+, 4 z-, 5 z+), or kNoTile
+    uint32_t    pad[2];
+};
+struct Resident3Args {
+    ResTile3*       rtile;   // [tiles] by rank
+    uint32_t*       seeds;   // [n_seeds]
+    uint32_t        n_seeds, tiles;
+    float           eps;
+    uint32_t*       edges;
+    unsigned long long* state;
+    uint32_t*       cmd;
+    uint32_t*       ctl;
+    unsigned long long* report;
+    HostRec*        rec;
+    uint32_t        tag;
+};
+constexpr uint32_t kRes3MaxGroups = 512;
+struct Resident3Kernel {
+    hipError_t (*launch)(const Resident3Args&, hipStream_t, hipEvent_t ev0, hipEvent_t ev1);
+    hipError_t (*init)(const Resident3Args&, const GhcmInst* h_inst, const uint32_t* h_seeds, hipStream_t);
+    int (*blocks_per_cu)();
+};
+Resident3Kernel get_resident3_kernel(int kind);
 
 }  // namespace ghcm

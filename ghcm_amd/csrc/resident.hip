@@ -343,7 +343,7 @@ void k_resident_sweep(ResidentArgs a) {
                     default: sweep_round<TW, TH, -1, false, kEvery, kSweepRound>(shb, L, exchange); break;
                 }
                 ++rounds;
-                const bool stop = (rounds & 1023u) == 0u && ld_agent(&a.cmd[b]) == kCmdAbort;
+                const bool stop = (rounds & 1023u) == 0u && must_stop(a.ctl, a.cmd, b, N, t_start);
                 uint32_t r = any4((__ballot(ch) ? 1u : 0u) | (__ballot(stop) ? 4u : 0u));
                 if (!(r & 1u)) {
                     pub = true;
@@ -583,7 +583,7 @@ void k_resident_sweep(ResidentArgs a) {
             sum_cells += red[kSweepThreads + i];
             most = max(most, (uint32_t)red[2 * kSweepThreads + i]);
         }
-        report_totals(a, sum_rounds, sum_rounds, sum_cells, most);
+        report_totals(a, sum_rounds, sum_rounds, sum_cells, most, !go || ld_agent(&a.ctl[kResFailed]) != 0u);
     }
 }
 

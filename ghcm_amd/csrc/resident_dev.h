@@ -51,16 +51,17 @@ __device__ __forceinline__ void resident_tile(const GhcmInst& in, uint32_t rank,
 }
 
 // A tile's record as wave-uniform values.
-__device__ __forceinline__ ResTile uniform_tile(const ResTile* p) {
-    static_assert(sizeof(ResTile) % 16 == 0, "whole vectors");
-    ResTile d;
+template <typename Tile>
+__device__ __forceinline__ Tile uniform_tile(const Tile* p) {
+    static_assert(sizeof(Tile) % 16 == 0, "whole vectors");
+    Tile d;
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 v[sizeof(ResTile) / 16];
+    u32x4 v[sizeof(Tile) / 16];
     uint32_t* const o = reinterpret_cast<uint32_t*>(&d);
 #pragma unroll
-    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) v[i] = gmem(reinterpret_cast<const u32x4*>(p))[i];
+    for (size_t i = 0; i < sizeof(Tile) / 16; ++i) v[i] = gmem(reinterpret_cast<const u32x4*>(p))[i];
 #pragma unroll
-    for (size_t i = 0; i < sizeof(ResTile) / 16; ++i) {
+    for (size_t i = 0; i < sizeof(Tile) / 16; ++i) {
         o[4 * i] = __builtin_amdgcn_readfirstlane(v[i].x);
         o[4 * i + 1] = __builtin_amdgcn_readfirstlane(v[i].y);
         o[4 * i + 2] = __builtin_amdgcn_readfirstlane(v[i].z);
@@ -84,23 +85,36 @@ __device__ __forceinline__ bool decide(uint32_t* ctl, uint32_t what) {
     return __hip_atomic_compare_exchange_strong(&ctl[kResDecision], &expect, what, __ATOMIC_RELAXED,
                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// 1 once every work-group is running; 2, and the solve given up, if that takes kJoinTicks.
+// 1 once every work-group is running; 2, the solve given up, if that takes kJoinTicks.
 __device__ __forceinline__ uint32_t await_decision(uint32_t* ctl, uint64_t t_start) {
     uint32_t d;
     while ((d = ld_agent(&ctl[kResDecision])) == 0u) {
-        if (now_ticks() - t_start > kJoinTicks && decide(ctl, 2u)) st_agent(&ctl[kResFailed], 1u);
+        if (now_ticks() - t_start > kJoinTicks) (void)decide(ctl, 2u);
         __builtin_amdgcn_s_sleep(4);
     }
     return d;
 }
 
-// The totals for the host, by one thread; the tag last.
-__device__ __forceinline__ void report_totals(const ResidentArgs& a, unsigned long long visits,
-                                              unsigned long long passes, unsigned long long cells, uint32_t most) {
+// Every 1,024 rounds a busy work-group asks whether to stop: told so, or out of time, in which case
+// it tells the others (N command words) and fails the solve.  Sweeps end by themselves (every round
+// but the last lowers a cell); this bounds them whatever the field holds.
+__device__ __forceinline__ bool must_stop(uint32_t* ctl, uint32_t* cmd, uint32_t own, uint32_t N, uint64_t t_start) {
+    if (ld_agent(&cmd[own]) == kCmdAbort) return true;
+    if (now_ticks() - t_start <= kLimitTicks) return false;
+    st_agent(&ctl[kResFailed], 1u);
+    for (uint32_t i = 0; i < N; ++i) st_agent(&cmd[i], kCmdAbort);
+    return true;
+}
+
+// The totals for the host, by one thread; the tag last.  failed: the solve was given up.
+template <typename Args>
+__device__ __forceinline__ void report_totals(const Args& a, unsigned long long visits,
+                                              unsigned long long passes, unsigned long long cells, uint32_t most,
+                                              bool failed) {
     sys_store64(&a.rec->totals[0], visits);
     sys_store64(&a.rec->totals[1], passes);
     sys_store64(&a.rec->totals[2], cells);
-    sys_store(&a.rec->wave, ld_agent(&a.ctl[kResFailed]));
+    sys_store(&a.rec->wave, failed ? 1u : 0u);
     sys_store(&a.rec->busy_waves, most);
     wait_stores();
     sys_store(&a.rec->totals_tag, a.tag);

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
             }
             __syncthreads();
         }
-        if (tid == 0) report_totals(a, red[0][0], red[0][0], red[1][0], (uint32_t)red[2][0]);
+        if (tid == 0) report_totals(a, red[0][0], red[0][0], red[1][0], (uint32_t)red[2][0], !go || ld_agent(&a.ctl[kResFailed]) != 0u);
         return;
     }
     const uint32_t rank = blockIdx.x + (uint32_t)(tid >> 6) * G;
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
                 }
                 publish();
                 more |= take();
-                if ((visits & 4095u) == 0u && ld_agent(&a.cmd[rank]) == kCmdAbort) break;
+                if ((visits & 1023u) == 0u && __ballot(must_stop(a.ctl, a.cmd, rank, T, t_start))) break;
                 if (!more) break;
             }
             work = false;
