@@ -51,7 +51,7 @@ __host__ __device__ constexpr uint32_t inbox_side(int s) {
 }  // namespace
 
 template <int TW, int TH, int KIND>
-__global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
+__device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
     constexpr int R = lane_rows<TW, TH>();
     // Passes between two looks, about one look's latency: for 8x8 tiles 2, 4, 6, 9 and 14 of them
     // 1,531, 1,318, 1,340, 1,466 and 1,610 us (512^2 rings), for 16x16 1, 2, 3, 5 and 8 582, 455,
@@ -350,20 +350,39 @@ __global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
 }
 
 template <int TW, int TH, int KIND>
+__global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
+    resident_wave<TW, TH, KIND>(a);
+}
+// 8x8 tiles, in at most 80 scalar registers: a SIMD has 800, handed out by 16, and 16 of each wave's
+// are the trap handler's, so 80 let eight waves run on it and the 88 that the compiler takes by
+// itself only seven -- three of these work-groups per CU instead of four, which the occupancy query
+// does not know: grids of 6,137 to 8,184 tiles joined too few and went to the wave loop (640^2 to
+// 744 x 704: 2,770-3,390 us; now 700-850).  The larger tiles' vector registers allow six at most.
+template <int KIND>
+__global__ __launch_bounds__(kWaveGroup) __attribute__((amdgpu_num_sgpr(80))) void k_resident_wave8(ResidentArgs a) {
+    resident_wave<8, 8, KIND>(a);
+}
+template <int TW, int TH, int KIND>
+constexpr auto wave_kernel() {
+    if constexpr (TW == 8 && TH == 8) return &k_resident_wave8<KIND>;
+    else return &k_resident_wave<TW, TH, KIND>;
+}
+
+template <int TW, int TH, int KIND>
 static hipError_t launch_wave_t(const ResidentArgs& a, uint32_t groups, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     if (a.tiles == 0 || a.tiles > kResMaxWaveTiles || groups != (a.tiles + kTilesPerGroup - 1) / kTilesPerGroup)
         return hipErrorInvalidValue;
     if (ev0 && ev1)
-        hipExtLaunchKernelGGL((k_resident_wave<TW, TH, KIND>), dim3(groups + 1), dim3(kWaveGroup), 0, s, ev0, ev1, 0, a);
+        hipExtLaunchKernelGGL((wave_kernel<TW, TH, KIND>()), dim3(groups + 1), dim3(kWaveGroup), 0, s, ev0, ev1, 0, a);
     else
-        hipLaunchKernelGGL((k_resident_wave<TW, TH, KIND>), dim3(groups + 1), dim3(kWaveGroup), 0, s, a);
+        hipLaunchKernelGGL((wave_kernel<TW, TH, KIND>()), dim3(groups + 1), dim3(kWaveGroup), 0, s, a);
     return hipGetLastError();
 }
 
 template <int TW, int TH, int KIND>
 static int occ_wave_t() {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_resident_wave<TW, TH, KIND>, kWaveGroup, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, wave_kernel<TW, TH, KIND>(), kWaveGroup, 0) != hipSuccess)
         return 0;
     return nb;
 }
