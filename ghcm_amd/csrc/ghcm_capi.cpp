@@ -695,6 +695,37 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
     // 16x16 FIM tiles 3,837 -> 455 us.
     bool resident_done = false;
+    // The events that stamp a resident launch, when kernels are profiled.
+    auto prof_events = [&](hipEvent_t* e0, hipEvent_t* e1) -> int {
+        if (!cfg.profile_kernels) return GHCM_OK;
+        while (ctx->ev_prof.size() < 2) {
+            hipEvent_t ev;
+            HIP_TRY(hipEventCreate(&ev));
+            ctx->ev_prof.push_back(ev);
+        }
+        *e0 = ctx->ev_prof[0];
+        *e1 = ctx->ev_prof[1];
+        return GHCM_OK;
+    };
+    // Waits for a resident solve; one that was given up before it began is left to the wave loop.
+    auto await_resident = [&](uint32_t tag, hipEvent_t e0, hipEvent_t e1) -> int {
+        HIP_TRY(hipEventRecord(ctx->ev_end, st));
+        if (int r = await_totals(tag)) return r;
+        if (hr->wave != 0) {
+            totals_ready = false;
+            return GHCM_OK;
+        }
+        resident_done = true;
+        converged = true;
+        waves_done = hr->busy_waves;
+        if (e0) {
+            float ms = 0.0f;
+            HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+            kern_us = 1000.0 * ms;
+            kern_launches = 1;
+        }
+        return GHCM_OK;
+    };
     const uint32_t cus = (uint32_t)std::max(1, ctx->cus);
     if (!three_d && !host_sched && !noalloc && cfg.launch_mode == 0 && cfg.max_waves == 0 && n_sel >= cus) {
         const ResidentKernel rk = get_resident_kernel((int)tw, (int)th, kind, cfg.kernel);
@@ -741,33 +772,53 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
             ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
             ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
             ra.tag = ++ctx->solve_seq;
-            const bool prof = cfg.profile_kernels != 0;
-            while (prof && ctx->ev_prof.size() < 2) {
-                hipEvent_t ev;
-                HIP_TRY(hipEventCreate(&ev));
-                ctx->ev_prof.push_back(ev);
-            }
-            const hipEvent_t e0 = prof ? ctx->ev_prof[0] : nullptr, e1 = prof ? ctx->ev_prof[1] : nullptr;
+            hipEvent_t e0 = nullptr, e1 = nullptr;
+            if ((rc = prof_events(&e0, &e1))) return rc;
             const GhcmInst* const inst_view = ctx->h_inst.dev_as<GhcmInst>();
             const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
             HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, seeds_view, groups, kind, st)
                               : wk.init(ra, inst_view, seeds_view, kind, st));
             HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
-            HIP_TRY(hipEventRecord(ctx->ev_end, st));
-            if ((rc = await_totals(ra.tag))) return rc;
-            if (hr->wave == 0) {
-                resident_done = true;
-                converged = true;
-                waves_done = hr->busy_waves;
-                if (prof) {
-                    float ms = 0.0f;
-                    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-                    kern_us = 1000.0 * ms;
-                    kern_launches = 1;
-                }
-            } else {
-                totals_ready = false;       // given up before it began: the wave loop solves it
-            }
+            if ((rc = await_resident(ra.tag, e0, e1))) return rc;
+        }
+    }
+    // 3-D sweep tiles (resident3.hip), up to one tile per resident work-group: 150 x 90 x 61 (288
+    // tiles) 888 -> 432 us; with several tiles each the wave loop is the better one (256^3 3,910
+    // against 6,430 us).
+    if (sweep3 && n_inst == 1 && cfg.launch_mode == 0 && cfg.max_waves == 0 && n_sel >= cus) {
+        const Resident3Kernel rk = get_resident3_kernel(kind);
+        const uint64_t fit = (uint64_t)std::max(0, rk.launch ? rk.blocks_per_cu() : 0) * cus;
+        if (rk.launch && T <= std::min<uint64_t>(fit, kRes3MaxGroups)) {
+            Resident3Args ra{};
+            ra.tiles = T;
+            ra.eps = cfg.min_change;
+            ra.n_seeds = (uint32_t)n_seeds_total;
+            ra.rec = ctx->rec.dev_as<HostRec>();
+            size_t need = 0;
+            auto part = [&need](size_t bytes) {
+                const size_t at = need;
+                need += (bytes + 255) & ~size_t(255);
+                return at;
+            };
+            const size_t o_edges = part(4ull * kRes3Words * T),
+                         o_tile = part(sizeof(ResTile3) * (size_t)T), o_state = part(8ull * kRes3MaxGroups),
+                         o_report = part(8ull * kRes3MaxGroups), o_cmd = part(4ull * kRes3MaxGroups),
+                         o_ctl = part(4ull * kResCtlWords), o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
+            if ((rc = ctx->resident.reserve(need))) return rc;
+            char* const base = ctx->resident.as<char>();
+            ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
+            ra.rtile = reinterpret_cast<ResTile3*>(base + o_tile);
+            ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
+            ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
+            ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
+            ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
+            ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
+            ra.tag = ++ctx->solve_seq;
+            hipEvent_t e0 = nullptr, e1 = nullptr;
+            if ((rc = prof_events(&e0, &e1))) return rc;
+            HIP_TRY(rk.init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
+            HIP_TRY(rk.launch(ra, st, e0, e1));
+            if ((rc = await_resident(ra.tag, e0, e1))) return rc;
         }
     }
     if (!resident_done && (rc = enqueue_init())) return rc;

@@ -98,7 +98,8 @@ typedef struct ghcm_config {
                                        wave (default; 64x64 sweep tiles, and grids of up to
                                        8,184 systolic or FIM tiles, with n of at least one
                                        tile per CU and no wave cap are solved by one
-                                       resident launch instead, without waves),
+                                       resident launch instead, without waves; so are
+                                       volumes of up to 512 sweep tiles),
                                        1 = one persistent cooperative launch runs every
                                        wave where built (sweep kernel; its grid barrier
                                        pays agent-scope fences),
@@ -208,7 +209,8 @@ int ghcm_solve_device_noalloc(ghcm_ctx* ctx, const void* d_field, int field_kind
  * `field` and the time are W*H*D cells, idx = x + W*(y + H*z); `seeds_xyz` holds
  * n_seeds (x, y, z) triples (host memory).  kernel GHCM_KERNEL_SWEEP solves 64x8x8
  * tiles with the eight octant sweeps (inner_iter_cap counts rounds of all eight), the
- * other kernels 8x8x8 tiles with in-tile passes; the device scheduler runs the wave loop:
+ * other kernels 8x8x8 tiles with in-tile passes; the device scheduler runs the wave loop,
+ * or the one resident launch of launch_mode 0:
  * n_active, min_change, inner_iter_cap, waves_per_poll, max_waves and launch_mode 2
  * (graph replay) apply, the tile shape fields do not (stats report tile_w/h/d), and
  * the host scheduler returns GHCM_ERR_UNSUPPORTED.  Host-buffer and device-buffer forms

@@ -12,6 +12,7 @@ import pytest
 
 import ghcm_amd as g
 import oracle
+from conftest import fixed_point_gap3d, ulp32
 from test_gpu_parity import check
 
 pytestmark = pytest.mark.gpu
@@ -105,6 +106,28 @@ def test_one_wave_tiles_storage_and_batch(rng, kind):
             check(t.download(), oracle.fmm_f32(c, q), q, c, label=f"{kind} {c.shape}", eps=0.0)
             d.free()
             t.free()
+
+
+# partial tiles in each axis, one cell, one tile row; 511 and 513 tiles (512 fit: above, wave loop)
+@pytest.mark.parametrize("kind", ["cost", "speed_f16"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (5, 3, 64), (8, 8, 65), (9, 17, 130), (30, 41, 70), (56, 584, 5), (24, 1368, 7)])
+def test_volumes(rng, shape, kind):
+    speed = rng.uniform(0.2, 5.0, shape)
+    stored = speed.astype(np.float16) if kind == "speed_f16" else (1.0 / speed).astype(np.float32)
+    cost = (1.0 / stored.astype(np.float32)).astype(np.float32) if kind == "speed_f16" else stored
+    d, h, w = shape
+    seeds = sorted({(0, 0, 0), (w - 1, h - 1, d - 1), (min(63, w - 1), min(7, h - 1), min(8, d - 1))})
+    print(f"case resident volume {shape} {kind}", flush=True)
+    ref = oracle.fmm3d_f64(cost, seeds)
+    with g.Context(0, **dict(CFG, n_active=2048)) as ctx:
+        for _ in range(2):
+            t, st = ctx.solve3d(stored, seeds, kind=g.KINDS[kind])
+            assert st["converged"] == 1
+            assert np.array_equal(np.isfinite(t), np.isfinite(ref))
+            # 1e-4 max T as in the 3-D parity tests, plus the least change that counts
+            assert float(np.max(np.abs(t - ref))) <= 1e-4 * float(ref.max()) + 1e-5
+            gap = fixed_point_gap3d(t, cost, seeds)
+            assert np.all(gap <= 4 * ulp32(t) + 2e-5), gap.max()
 
 
 def test_no_seeds_and_walled_off_tiles():
