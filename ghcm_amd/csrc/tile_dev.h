@@ -210,7 +210,7 @@ __device__ __forceinline__ void sweep_round(char* const shb, const int L, F betw
     // advances by one row per step, back to the first row exactly there (the wrap of the row
     // index coincides with the pass start).
     constexpr uint64_t kFirstPat = TH >= 64 ? 1ull : ~0ull / ((1ull << (TH & 63)) - 1ull);
-    constexpr int SE = (STEPS + 1) & ~1;
+    constexpr int SE = (STEPS + 3) & ~3;
     int bb = b_start - b_step;
     uint32_t jl = 0;
     struct Nb {
@@ -219,9 +219,12 @@ __device__ __forceinline__ void sweep_round(char* const shb, const int L, F betw
         bool first;
     };
     auto at = [&](int b, int word) -> float { return *reinterpret_cast<const float*>(shb + b + 4 * word); };
-    // LDS reads of step s+1 are issued before step s is computed (two register sets): their
-    // cells are upper bounds whatever the interleaving, and the fresh upwind values arrive
-    // through DPP and `prev`, so the dependent chain per step is DPP + update.
+    // LDS reads of step s+1 are issued before step s is computed: their cells are upper bounds
+    // whatever the interleaving, and the fresh upwind values arrive through DPP and `prev`, so the
+    // dependent chain per step is DPP + update.  Four register sets in rotation: with two, the reads
+    // of step s+1 wait for the registers that step s-1 still uses (whole resident solves with two ->
+    // four: 256^2 rings 232 -> 219 us, 1531 x 977 smooth 337 -> 315, 2048^2 contrast 1,750 -> 1,600;
+    // reads two or three steps ahead are no faster, 320 and 1,660 us, and slower where the CU is full).
     auto load = [&](Nb& o) {
         o.first = __builtin_amdgcn_inverse_ballot_w64(kFirstPat << (jl & (TH - 1)));
         ++jl;
@@ -249,30 +252,22 @@ __device__ __forceinline__ void sweep_round(char* const shb, const int L, F betw
         // their own LDS read of the cell.
         prev = t;
     };
-    Nb A, B;
-    load(A);
-    if constexpr (CHUNK == 0) {
-#pragma unroll 2
-        for (int st = 0; st < SE; st += 2) {
-            load(B);
+    Nb X[4];
+    load(X[0]);
+    auto four = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            load(X[(i + 1) & 3]);
             __builtin_amdgcn_sched_barrier(0);
-            step(A);
-            load(A);
-            __builtin_amdgcn_sched_barrier(0);
-            step(B);
+            step(X[i]);
         }
+    };
+    if constexpr (CHUNK == 0) {
+        for (int st = 0; st < SE; st += 4) four();
     } else {
-        static_assert(SE % CHUNK == 0 && CHUNK % 2 == 0, "whole chunks");
+        static_assert(SE % CHUNK == 0 && CHUNK % 4 == 0, "whole chunks");
         for (int ch = 0; ch < SE / CHUNK; ++ch) {
-#pragma unroll 2
-            for (int st = 0; st < CHUNK; st += 2) {
-                load(B);
-                __builtin_amdgcn_sched_barrier(0);
-                step(A);
-                load(A);
-                __builtin_amdgcn_sched_barrier(0);
-                step(B);
-            }
+            for (int st = 0; st < CHUNK; st += 4) four();
             between();
         }
     }
