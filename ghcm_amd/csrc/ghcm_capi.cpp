@@ -685,11 +685,10 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // whose n fills the chip (at least one tile per CU: the wave loop cuts below that, and a
     // caller that sets n small asks for the cut) and no wave cap, and up to 256 tiles per
     // resident work-group (262,144 tiles on 256 CUs).  2048^2 (one tile each) 1,020 -> 540 us,
-    // 4096^2 (four) 1,774 -> 970 us, a batch of 512 (143) 20.9 -> 13.3 ms.
-    // Up to kScanOwned tiles each, work-groups scan the borders of their closed tiles, above it
-    // they are told: four tiles 1,020 against 1,180 us, eight 1,400 against 1,550, 21 3.76
-    // against 3.38 ms.
-    constexpr uint32_t kScanOwned = 8;
+    // 4096^2 (four) 1,774 -> 1,020 us, a batch of 512 (143) 20.9 -> 11.8 ms.
+    // Up to kResMaxScan tiles each, work-groups scan the borders of their closed tiles, above it
+    // they are told: four tiles 1,040 against 1,130 us, eight 2,080 against 2,260, eleven 3,015
+    // against 3,300, 15 equal, a batch of 21 each 3,600 against 3,110.
     // The one-wave tiles (resident_wave.hip) likewise, one wave64 per tile with the tile in
     // registers, up to the resident waves (8,184 tiles of 8x8 or 6,136 of 16x16 on 256 CUs; larger
     // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
@@ -738,7 +737,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                                     : wk.launch && T <= kResMaxWaveTiles && groups + 1u <= fit;
         if (fits) {
             const uint32_t owned = rk.launch ? (T + groups - 1) / groups : 1u;
-            const bool scan = owned <= kScanOwned;
+            const bool scan = owned <= kResMaxScan;
             const uint32_t states = rk.launch ? kResMaxGroups : kResMaxWaveTiles;
             ResidentArgs ra{};
             ra.n_inst = n_inst;

@@ -20,7 +20,7 @@ enum : uint32_t {
 };
 
 constexpr uint32_t kResMaxGroups = 1024;     // work-groups whose states one of them watches
-constexpr uint32_t kResMaxScan = 32;         // tiles of one work-group that scans their borders
+constexpr uint32_t kResMaxScan = 16;         // tiles of one work-group that scans their borders
 constexpr uint32_t kResMaxOwned = 256;       // tiles of one work-group (one want a thread)
 
 // What a work-group needs to open a tile: one read.
@@ -34,7 +34,8 @@ struct alignas(16) ResTile {
     uint32_t    face[4];     // across side s: id * 4 + side of the border facing it, or kNoTile
     uint32_t    call[4];     // and where in `want` its owner is told
     uint32_t    x0, y0;      // its origin
-    uint32_t    pad[2];
+    float       pace;        // 1 / (tiles across and down its grid): times by it are compared in `want`
+    uint32_t    pad;
 };
 
 struct ResidentArgs {
@@ -47,7 +48,7 @@ struct ResidentArgs {
     uint32_t*       edges;   // [tiles][4][64] published border cells (float bits), side-major
     // With several tiles to a work-group, one of (the other null):
     uint32_t*       seen;    // [tiles][4][64] the neighbours' facing borders a closed tile was left with
-    uint32_t*       want;    // [groups][want_stride] smallest new border value of an owned tile's neighbours
+    uint32_t*       want;    // [groups][want_stride] smallest new border value of an owned tile's neighbours, by pace
     uint32_t        want_stride;
     unsigned long long* state;  // [groups] (acknowledged epoch << 32) | visit counter, odd while busy
     uint32_t*       cmd;     // [groups] epoch to acknowledge, or kCmdDone / kCmdAbort

@@ -30,7 +30,10 @@
 //              closed tiles against seen[], what they were when it closed them; with many, who
 //              publishes a border then lowers want[] of the tile across, which the owner reads
 //              in one load for all its tiles and withdraws before it reads the borders: what is
-//              announced after that the looks at the then open tile see.
+//              announced after that the looks at the then open tile see.  Wants are times over
+//              the tiles across the grid, so that the small and the large instances of a batch
+//              advance alike (a batch of 512 12.1 -> 11.8 ms; the largest instances first, which
+//              would shorten the end, 14.7 ms: tiles are then opened before all of a front is in).
 //   end        a work-group publishes a counter that is odd while it works: odd before its
 //              first border store is issued, even after its last one is visible.  Work-group 0,
 //              when idle, reads all counters; if all are even it sends an epoch, which a
@@ -42,10 +45,13 @@
 //              takes over 200 us (other work holds the CUs) all leave at once and the caller runs
 //              the wave loop.  Every wait ends: on the decision, on the end or on a 20 s limit.
 //
-// Measured (MI355X, whole calls, wave loop -> this): 256^2 rings 452 -> 231 us, 1531 x 977 smooth
-// 813 -> 339, 2048^2 rings of contrast 1e4 4300 -> 1745, 2048^2 smooth 1020 -> 540, 4096^2
-// smooth 1774 -> 1050, a batch of 48 uneven fields (1,123 tiles) 845 -> 400,
-// a batch of 512 (147 k tiles) 20.9 -> 13.3 ms.
+// Measured (MI355X, whole calls, wave loop -> this): 256^2 rings 452 -> 217 us, 1531 x 977 smooth
+// 813 -> 315, 2048^2 rings of contrast 1e4 4300 -> 1600, 2048^2 smooth 1020 -> 520, 4096^2
+// smooth 1774 -> 1020, a batch of 48 uneven fields (1,123 tiles) 845 -> 390, a batch of 512 (147 k
+// tiles) 20.9 -> 11.8 ms.  There each SIMD has the sweeps of four work-groups to issue (15 vector
+// instructions and a square root a step) and is busy three quarters of the time.  Taken back:
+// sweeping only the directions that the new border values or the unsettled cells ask for (12 %
+// more rounds, and each as long as the latency of its steps, 12.4 against 11.9 ms).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -64,15 +70,25 @@ namespace {
 // (never closed), it scans the borders that face them all, or their neighbours' owners tell it.
 enum : int { kOwnOne = 0, kOwnScan = 1, kOwnWant = 2 };
 
-// Sweep steps between two exchanges: 8 against 16 and 32, 4096^2 1,050 against 1,100 and 1,430 us,
-// 2048^2 contrast 1,800 against 1,870 and 2,400 us, smaller grids equal.
+// Sweep steps between two exchanges: 8 against 16 and 32, 2048^2 contrast 1,800 against 1,870 and
+// 2,400 us, smaller grids equal.
 constexpr int kChunk = 8;
-// With many tiles to a work-group all CUs are busy and a front is no longer waited for: a batch of
-// 512 uneven fields 13.3 ms at 16, 13.9 at 8.
-constexpr int kChunkWant = 16;
+// With several tiles to a work-group the CUs are busy and a front is no longer waited for: 4096^2
+// (four tiles each) 1,020 us at 16, 1,140 at 8, 1,280 at 32; a batch of 512 uneven fields (143)
+// 11.8 ms at 16 and 32, 12.3 at 8.
+constexpr int kChunkMany = 16;
 // Sweep steps of a round: one ordered pass of all lanes (127) rounded up to the period of the
 // wrapped skew, so that the next round takes up where this one ended.
 constexpr int kSweepRound = 128;
+// With several tiles to a work-group only the first round on a tile's new borders is that long and
+// those after it half as long, one period of the skew: what is left to lower is little, and the
+// sweeps of all the CU's work-groups share its issue slots.  Whole against half later rounds: 4096^2
+// 1,130 against 1,020 us, 40 fields of up to 1200^2 1,910 against 1,700, the batch of 512 13.0
+// against 11.9 ms; all rounds half 12.1 ms, and with one tile each 1531 x 977 355 against 338 us.
+constexpr int kManyParts = 2;
+// The largest `want` of a tile that is wanted (a product of finite times may overflow).
+constexpr float kLatest = 3e38f;
+
 // OR of `bits` over the four waves; one barrier.  Consecutive calls use different buffers.
 __device__ __forceinline__ uint32_t wg_or(uint32_t bits, uint32_t* buf, int w, int L) {
     if (L == 0) buf[w] = bits;
@@ -87,7 +103,9 @@ __global__ __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(4
 void k_resident_sweep(ResidentArgs a) {
     constexpr int PW = TW + 2, PH = TH + 2, PP = PW * PH, CB = PP + 1;
     constexpr int CPT = TW * TH / kSweepThreads;
-    constexpr int kEvery = OWN == kOwnWant ? kChunkWant : kChunk;
+    constexpr int kEvery = OWN == kOwnOne ? kChunk : kChunkMany;
+    constexpr int kParts = OWN == kOwnOne ? 1 : kManyParts, kSteps = kSweepRound / kParts;
+    static_assert(kSteps % TH == 0, "a part takes up where the one before ended");
     __shared__ float sh[sweep_lds_words<TW, TH>()];
     __shared__ uint32_t s_or[3][4];
     __shared__ uint32_t s_cmd[2];
@@ -155,6 +173,7 @@ void k_resident_sweep(ResidentArgs a) {
     int q_own = PW + 1, q_halo = 0;
     const uint32_t* from = a.edges;
     uint32_t* to = a.edges;
+    float pace = 0.0f;                  // of the tile's times in `want`
     uint32_t* call = nullptr;           // the want of the tile across this side
     float halo = __builtin_inff();      // the neighbour's border cell, as last read
     float sent = __builtin_inff();      // this tile's border cell, as last published
@@ -219,7 +238,10 @@ void k_resident_sweep(ResidentArgs a) {
         act = nact;
         from = nfrom;
         to = nto;
-        if constexpr (OWN == kOwnWant) call = a.want + told;
+        if constexpr (OWN == kOwnWant) {
+            call = a.want + told;
+            pace = d.pace;
+        }
         halo = nhalo;
         sent = nsent;
         // box words of lane L's border cell and of the halo cell across this side
@@ -304,7 +326,7 @@ void k_resident_sweep(ResidentArgs a) {
                     sent = mine;
                 }
                 if (OWN == kOwnWant && __ballot(out))
-                    key = min(key, __float_as_uint(wave_min(out ? mine : __builtin_inff())));
+                    key = min(key, __float_as_uint(fminf(pace * wave_min(out ? mine : __builtin_inff()), kLatest)));
             };
             auto exchange = [&]() {
                 const float v = ahead;
@@ -332,16 +354,20 @@ void k_resident_sweep(ResidentArgs a) {
             };
             // Rounds go on while they bring new halo values; after one that brought none, the
             // box is checked cell by cell.
+            bool first = true;
             do {
                 ch = false;
                 // The open tile's neighbours announce what the exchanges see by themselves.
                 if (OWN == kOwnWant && tid == 0) st_agent(&want[cur], kInfBits);
-                switch (w) {
-                    case 0: sweep_round<TW, TH, 1, true, kEvery, kSweepRound>(shb, L, exchange); break;
-                    case 1: sweep_round<TW, TH, -1, true, kEvery, kSweepRound>(shb, L, exchange); break;
-                    case 2: sweep_round<TW, TH, 1, false, kEvery, kSweepRound>(shb, L, exchange); break;
-                    default: sweep_round<TW, TH, -1, false, kEvery, kSweepRound>(shb, L, exchange); break;
+                for (int part = first ? 0 : kParts - 1; part < kParts; ++part) {
+                    switch (w) {
+                        case 0: sweep_round<TW, TH, 1, true, kEvery, kSteps>(shb, L, exchange); break;
+                        case 1: sweep_round<TW, TH, -1, true, kEvery, kSteps>(shb, L, exchange); break;
+                        case 2: sweep_round<TW, TH, 1, false, kEvery, kSteps>(shb, L, exchange); break;
+                        default: sweep_round<TW, TH, -1, false, kEvery, kSteps>(shb, L, exchange); break;
+                    }
                 }
+                first = false;
                 ++rounds;
                 const bool stop = (rounds & 1023u) == 0u && must_stop(a.ctl, a.cmd, b, N, t_start);
                 uint32_t r = any4((__ballot(ch) ? 1u : 0u) | (__ballot(stop) ? 4u : 0u));

@@ -174,7 +174,8 @@ __global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const ui
                 const uint32_t r = nb == kNoTile ? 0u : resident_rank(in, (uint32_t)(tx + side_dx(s)), (uint32_t)(ty + side_dy(s)));
                 d.call[s] = (r % N) * a.want_stride + r / N;
             }
-            d.pad[0] = d.pad[1] = 0u;
+            d.pace = 1.0f / (float)(in.tiles_x + in.tiles_y);
+            d.pad = 0u;
             a.rtile[in.tile_base + t] = d;
         }
     }

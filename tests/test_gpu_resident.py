@@ -141,10 +141,11 @@ def test_no_seeds_and_walled_off_tiles():
     check(t, oracle.fmm_f32(cost, [(3, 3)]), [(3, 3)], cost)
 
 
-@pytest.mark.parametrize("n_inst", [7, 160, 900])
+@pytest.mark.parametrize("n_inst", [7, 160, 600, 900])
 def test_uneven_batch(rng, n_inst):
     """Several instances in one resident launch; 160 of them have more tiles than work-groups
-    (which scan the borders of their closed tiles), 900 over eight tiles to each (which are told)."""
+    (which scan the borders of their closed tiles), 600 about eleven tiles to each, 900 over 16
+    (which are told)."""
     shapes = [(int(rng.integers(1, 300)), int(rng.integers(1, 300))) for _ in range(n_inst - 1)] + [(300, 1400)]
     if n_inst > 100:
         shapes = [(h + 100, w + 100) for h, w in shapes]
