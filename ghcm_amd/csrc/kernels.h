@@ -62,12 +62,17 @@ hipError_t launch_reduce_stats(const uint32_t* tstat, uint32_t tiles, unsigned l
                               hipStream_t s);
 hipError_t launch_seed_serve(const SolveArgs& a, const uint32_t* seeds_xyi, uint32_t n_seeds,
                              uint32_t tile_w, uint32_t tile_h, hipStream_t s);
-// One admitted request: its slot entry, tile states and tile map, its time field at +INF and,
-// with tw != 0 (th rows per edge column, cost kind `kind`), its tiles' edge columns.
-hipError_t launch_admit_tiles(const SolveArgs& a, const GhcmInst& in, uint32_t slot,
-                              uint32_t gen, hipStream_t s, uint32_t tw = 0, uint32_t th = 0,
-                              int kind = 0);
-hipError_t launch_wake(GhcmCtrl* ctrl, hipStream_t s);
+// An admitted request.
+struct alignas(16) AdmitRec {
+    GhcmInst in;
+    uint32_t slot, gen;
+    uint32_t pad[2];
+};
+// n admitted requests (recs: device view of mapped host memory): the slot entries, tile states and
+// tile map, the time fields at +INF and, with tw != 0 (th rows per edge column, cost kind `kind`),
+// the tiles' edge columns; the loop leaves its idle state.  max_cells: of the largest.
+hipError_t launch_admit_tiles(const SolveArgs& a, const AdmitRec* recs, uint32_t n, uint64_t max_cells,
+                              hipStream_t s, uint32_t tw = 0, uint32_t th = 0, int kind = 0);
 // h_inst: device view of the mapped host instance table.  tw != 0: also the edge columns of
 // every instance's tiles (tw x th x td tiles, cost kind `kind`; nothing when a.edge is null).
 hipError_t launch_solve_init(const SolveArgs& a, const GhcmInst* h_inst, uint32_t n_inst,

@@ -3,12 +3,12 @@
 // One device wave loop runs for the lifetime of the server and never restarts between
 // requests.  A request is admitted between waves when an instance slot, a range of tile
 // state and (for host buffers) room for its field and time buffer inside the HBM arena
-// are all free, first come first served.  Admission is a few launches on the loop's
-// stream: the slot's instance entry, admission generation and tile range are reset
-// (k_admit_tiles), the time buffer is set to +INF, the seeds queue their tiles for the
-// next wave (k_seed_serve, as a plain solve's seeds are queued for its first wave,
-// src/eikonal_hcm.cpp:189-238) and the loop leaves its idle state (k_wake).  From then
-// on the request's tiles compete in the same top-n selection as every live request's.
+// are all free, first come first served.  Admission of all requests that fit is two launches
+// on the loop's stream: k_admit_tiles resets the slots' instance entries, admission
+// generations and tile ranges, sets the time buffers to +INF and wakes an idle loop, then
+// the seeds queue their tiles for the next wave (k_seed_serve, as a plain solve's seeds are
+// queued for its first wave, src/eikonal_hcm.cpp:189-238).  From then on the requests' tiles
+// compete in the same top-n selection as every live request's.
 //
 // Every wave boundary (k_wave_end) writes, into mapped pinned host memory, each slot's
 // queued-tile count tagged with the slot's generation.  A request is finished at the
@@ -209,10 +209,10 @@ struct ghcm_server {
     hipGraphExec_t gexec = nullptr;
     DevBuf arena, inst, tinst, qwave, key, mask, tmin, list, tstat, sel, ctrl, sgen, totals;
     DevBuf edge, cedge;                  // sweep kernel: edge columns of every tile of the pool
-    static constexpr int kSeedRing = 8;   // seed staging buffers, reused round robin
-    PinnedBuf h_seeds[kSeedRing], rec;
-    hipEvent_t ev_seed[kSeedRing] = {};  // recorded after the launch that read each buffer
-    int seed_next = 0;
+    static constexpr int kAdmitRing = 8;  // admissions' staging buffers, reused round robin
+    PinnedBuf h_admit[kAdmitRing], rec;
+    hipEvent_t ev_admit[kAdmitRing] = {};  // recorded after the launches that read each buffer
+    int admit_next = 0;
     PinnedPool pool;
     SolveArgs a{};
     RangeAlloc arena_alloc, tile_alloc;
@@ -294,9 +294,9 @@ int ghcm_server::init() {
         if ((rc = edge.reserve(8ull * th * T))) return rc;
         if ((rc = cedge.reserve(8ull * th * T))) return rc;
     }
-    for (int k = 0; k < kSeedRing; ++k) {
-        if ((rc = h_seeds[k].reserve(12 * 1024))) return rc;
-        HIP_TRY(hipEventCreateWithFlags(&ev_seed[k], hipEventDisableTiming));
+    for (int k = 0; k < kAdmitRing; ++k) {
+        if ((rc = h_admit[k].reserve(sizeof(AdmitRec) * slots + 12 * 1024))) return rc;
+        HIP_TRY(hipEventCreateWithFlags(&ev_admit[k], hipEventDisableTiming));
     }
 
     a.inst = inst.as<GhcmInst>();
@@ -372,10 +372,10 @@ void ghcm_server::release_all() {
     for (DevBuf* b : {&arena, &inst, &tinst, &qwave, &key, &mask, &tmin, &list, &tstat, &sel, &ctrl,
                       &sgen, &totals, &edge, &cedge})
         b->release();
-    for (int k = 0; k < kSeedRing; ++k) {
-        h_seeds[k].release();
-        if (ev_seed[k]) (void)hipEventDestroy(ev_seed[k]);
-        ev_seed[k] = nullptr;
+    for (int k = 0; k < kAdmitRing; ++k) {
+        h_admit[k].release();
+        if (ev_admit[k]) (void)hipEventDestroy(ev_admit[k]);
+        ev_admit[k] = nullptr;
     }
     rec.release();
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
@@ -454,17 +454,19 @@ int ghcm_server::admit(std::vector<Request*>& batch, uint32_t enqueued) {
         HIP_TRY(hipEventRecord(ev_upload, up_stream));
         HIP_TRY(hipStreamWaitEvent(stream, ev_upload, 0));
     }
-    // Seed staging: a ring of mapped buffers read by k_seed_serve; a buffer is reused once
-    // the launch that read it, kSeedRing admissions ago, has run.
-    const int ring = seed_next;
-    if (n_seeds) {
-        seed_next = (seed_next + 1) % kSeedRing;
-        HIP_TRY(ghcm_capi::spin_wait(ev_seed[ring]));
-        int rc = h_seeds[ring].reserve(12 * n_seeds);
-        if (rc) return rc;
-    }
-    uint32_t* hs = h_seeds[ring].as<uint32_t>();
+    // Staging: a ring of mapped buffers, the requests' records and then their seeds, read by
+    // k_admit_tiles and k_seed_serve; a buffer is reused once the launches that read it,
+    // kAdmitRing admissions ago, have run.
+    const int ring = admit_next;
+    const size_t seeds_at = sizeof(AdmitRec) * batch.size();
+    admit_next = (admit_next + 1) % kAdmitRing;
+    HIP_TRY(ghcm_capi::spin_wait(ev_admit[ring]));
+    if (int rc = h_admit[ring].reserve(seeds_at + 12 * n_seeds)) return rc;
+    AdmitRec* const recs = h_admit[ring].as<AdmitRec>();
+    uint32_t* const hs = reinterpret_cast<uint32_t*>(h_admit[ring].as<char>() + seeds_at);
     size_t k = 0;
+    uint32_t n = 0;
+    uint64_t max_cells = 0;
     for (Request* r : batch) {
         const uint64_t cells = (uint64_t)r->w * r->h;
         GhcmInst g{};
@@ -484,9 +486,8 @@ int ghcm_server::admit(std::vector<Request*>& batch, uint32_t enqueued) {
         g.tiles_z = 1;
         r->gen = next_gen++;
         if (next_gen == 0) next_gen = 1;
-        // The slot's entry, tile states and tile map, its time field at +INF and its tiles'
-        // edge columns (sweep kernel) in one launch.
-        HIP_TRY(launch_admit_tiles(a, g, r->slot, r->gen, stream, tw, th, kind));
+        recs[n++] = AdmitRec{g, r->slot, r->gen, {0u, 0u}};
+        max_cells = std::max(max_cells, cells);
         for (size_t s = 0; s + 1 < r->seeds.size(); s += 2) {
             hs[k++] = r->seeds[s];
             hs[k++] = r->seeds[s + 1];
@@ -496,11 +497,10 @@ int ghcm_server::admit(std::vector<Request*>& batch, uint32_t enqueued) {
         r->state = ReqState::Live;
         live[r->slot] = r;
     }
-    if (n_seeds) {
-        HIP_TRY(launch_seed_serve(a, h_seeds[ring].dev_as<uint32_t>(), (uint32_t)n_seeds, tw, th, stream));
-        HIP_TRY(hipEventRecord(ev_seed[ring], stream));
-    }
-    HIP_TRY(launch_wake(a.ctrl, stream));
+    HIP_TRY(launch_admit_tiles(a, h_admit[ring].dev_as<AdmitRec>(), n, max_cells, stream, tw, th, kind));
+    HIP_TRY(launch_seed_serve(a, reinterpret_cast<const uint32_t*>(h_admit[ring].dev_as<char>() + seeds_at),
+                              (uint32_t)n_seeds, tw, th, stream));
+    HIP_TRY(hipEventRecord(ev_admit[ring], stream));
     return GHCM_OK;
 }
 
