@@ -301,6 +301,7 @@ void k_resident_sweep(ResidentArgs a) {
     bool work = (OWN == kOwnOne || m == 1u) && (s_seeded[0] & 1u);
     while (go) {
         if (work) {
+            __builtin_amdgcn_s_setprio(kWorkPriority);
             if (!(st & 1u)) {
                 ++st;
                 if (tid == 0) st_agent64(&a.state[b], ((unsigned long long)acked << 32) | st);
@@ -393,6 +394,7 @@ void k_resident_sweep(ResidentArgs a) {
                 tell();
             }
             work = false;
+            __builtin_amdgcn_s_setprio(0);
         }
         // ---- look at every owned tile's neighbours ----
         bool idle = false;

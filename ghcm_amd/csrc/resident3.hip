@@ -183,6 +183,7 @@ void k_resident_sweep3(Resident3Args a) {
     bool work = any8(__ballot(seeded) ? 1u : 0u) != 0u;
     while (go) {
         if (work) {
+            __builtin_amdgcn_s_setprio(kWorkPriority);
             if (!(st & 1u)) {
                 ++st;
                 put_state();
@@ -246,6 +247,7 @@ void k_resident_sweep3(Resident3Args a) {
                 }
             } while (more);
             work = false;
+            __builtin_amdgcn_s_setprio(0);
         }
         bool idle = false;
         for (;;) {

@@ -278,6 +278,7 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
     };
     for (;;) {
         if (work) {
+            __builtin_amdgcn_s_setprio(kWorkPriority);
             least = 0.0f;
             bool visible = (st & 1u) != 0u;         // (the first counter is odd from the start)
             if (!(st & 1u)) {
@@ -303,6 +304,7 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
                 if (!more) break;
             }
             work = false;
+            __builtin_amdgcn_s_setprio(0);
             least = eps;
         }
         if (st & 1u) {
