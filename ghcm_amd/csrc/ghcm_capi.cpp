@@ -706,6 +706,13 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
         *e1 = ctx->ev_prof[1];
         return GHCM_OK;
     };
+    // The resident workspace; where it does not fit in what is left of the HBM, the wave loop
+    // solves without it.
+    auto resident_room = [&](size_t need) -> bool {
+        if (ctx->resident.reserve(need) == GHCM_OK) return true;
+        (void)hipGetLastError();
+        return false;
+    };
     // Waits for a resident solve; one that was given up before it began is left to the wave loop.
     auto await_resident = [&](uint32_t tag, hipEvent_t e0, hipEvent_t e1) -> int {
         HIP_TRY(hipEventRecord(ctx->ev_end, st));
@@ -759,26 +766,27 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                          o_tile = part(sizeof(ResTile) * (size_t)T), o_state = part(8ull * states),
                          o_report = part(8ull * states), o_cmd = part(4ull * states), o_ctl = part(4ull * kResCtlWords),
                          o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
-            if ((rc = ctx->resident.reserve(need))) return rc;
-            char* const base = ctx->resident.as<char>();
-            ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
-            if (owned > 1 && scan) ra.seen = reinterpret_cast<uint32_t*>(base + o_seen);
-            if (owned > 1 && !scan) ra.want = reinterpret_cast<uint32_t*>(base + o_want);
-            ra.rtile = reinterpret_cast<ResTile*>(base + o_tile);
-            ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
-            ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
-            ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
-            ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
-            ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
-            ra.tag = ++ctx->solve_seq;
-            hipEvent_t e0 = nullptr, e1 = nullptr;
-            if ((rc = prof_events(&e0, &e1))) return rc;
-            const GhcmInst* const inst_view = ctx->h_inst.dev_as<GhcmInst>();
-            const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
-            HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, seeds_view, groups, kind, st)
-                              : wk.init(ra, inst_view, seeds_view, kind, st));
-            HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
-            if ((rc = await_resident(ra.tag, e0, e1))) return rc;
+            if (resident_room(need)) {
+                char* const base = ctx->resident.as<char>();
+                ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
+                if (owned > 1 && scan) ra.seen = reinterpret_cast<uint32_t*>(base + o_seen);
+                if (owned > 1 && !scan) ra.want = reinterpret_cast<uint32_t*>(base + o_want);
+                ra.rtile = reinterpret_cast<ResTile*>(base + o_tile);
+                ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
+                ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
+                ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
+                ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
+                ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
+                ra.tag = ++ctx->solve_seq;
+                hipEvent_t e0 = nullptr, e1 = nullptr;
+                if ((rc = prof_events(&e0, &e1))) return rc;
+                const GhcmInst* const inst_view = ctx->h_inst.dev_as<GhcmInst>();
+                const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
+                HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, seeds_view, groups, kind, st)
+                                  : wk.init(ra, inst_view, seeds_view, kind, st));
+                HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
+                if ((rc = await_resident(ra.tag, e0, e1))) return rc;
+            }
         }
     }
     // 3-D sweep tiles (resident3.hip), up to one tile per resident work-group: 150 x 90 x 61 (288
@@ -803,21 +811,22 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                          o_tile = part(sizeof(ResTile3) * (size_t)T), o_state = part(8ull * kRes3MaxGroups),
                          o_report = part(8ull * kRes3MaxGroups), o_cmd = part(4ull * kRes3MaxGroups),
                          o_ctl = part(4ull * kResCtlWords), o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
-            if ((rc = ctx->resident.reserve(need))) return rc;
-            char* const base = ctx->resident.as<char>();
-            ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
-            ra.rtile = reinterpret_cast<ResTile3*>(base + o_tile);
-            ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
-            ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
-            ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
-            ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
-            ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
-            ra.tag = ++ctx->solve_seq;
-            hipEvent_t e0 = nullptr, e1 = nullptr;
-            if ((rc = prof_events(&e0, &e1))) return rc;
-            HIP_TRY(rk.init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
-            HIP_TRY(rk.launch(ra, st, e0, e1));
-            if ((rc = await_resident(ra.tag, e0, e1))) return rc;
+            if (resident_room(need)) {
+                char* const base = ctx->resident.as<char>();
+                ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
+                ra.rtile = reinterpret_cast<ResTile3*>(base + o_tile);
+                ra.state = reinterpret_cast<unsigned long long*>(base + o_state);
+                ra.report = reinterpret_cast<unsigned long long*>(base + o_report);
+                ra.cmd = reinterpret_cast<uint32_t*>(base + o_cmd);
+                ra.ctl = reinterpret_cast<uint32_t*>(base + o_ctl);
+                ra.seeds = reinterpret_cast<uint32_t*>(base + o_seeds);
+                ra.tag = ++ctx->solve_seq;
+                hipEvent_t e0 = nullptr, e1 = nullptr;
+                if ((rc = prof_events(&e0, &e1))) return rc;
+                HIP_TRY(rk.init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
+                HIP_TRY(rk.launch(ra, st, e0, e1));
+                if ((rc = await_resident(ra.tag, e0, e1))) return rc;
+            }
         }
     }
     if (!resident_done && (rc = enqueue_init())) return rc;
