@@ -685,7 +685,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // whose n fills the chip (at least one tile per CU: the wave loop cuts below that, and a
     // caller that sets n small asks for the cut) and no wave cap, and up to 256 tiles per
     // resident work-group (262,144 tiles on 256 CUs).  2048^2 (one tile each) 1,020 -> 540 us,
-    // 4096^2 (four) 1,774 -> 1,020 us, a batch of 512 (143) 20.9 -> 11.8 ms.
+    // 4096^2 (four) 1,670 -> 950 us, a batch of 512 (143) 20.6 -> 10.3 ms.
     // Up to kResMaxScan tiles each, work-groups scan the borders of their closed tiles, above it
     // they are told: four tiles 1,040 against 1,130 us, eight 2,080 against 2,260, eleven 3,015
     // against 3,300, 15 equal, a batch of 21 each 3,600 against 3,110.

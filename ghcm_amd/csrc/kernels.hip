@@ -2306,8 +2306,8 @@ __device__ void sweep3_tile(const SolveArgs& a, uint32_t g, uint32_t wave, uint3
     for (;;) {
         // Wave w runs octant w: bit 0 -x, bit 1 -y, bit 2 -z (the branch is wave-uniform).
         // The sweeps, one chain of dependent steps, are issued before what the CU's other
-        // work-groups stage and commit: 256^3 3,565 -> 3,460 and 3,775 -> 3,704 us.  (The 2-D sweep kernel, whose
-        // waves are shorter than its launches, gains nothing by it; staging first: no gain.)
+        // work-groups stage and commit: 256^3 3,565 -> 3,460 and 3,775 -> 3,704 us.  (Staging
+        // first: no gain, and none of either in the 2-D sweep kernel.)
         __builtin_amdgcn_s_setprio(2);
         switch (w) {
             case 0: sweep3_round<1, 1, 1>(shb, L); break;
