@@ -200,33 +200,52 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
         }
     }
 
-    // One relaxation of cell k from its four neighbours; whether it improved by `least`: eps to
-    // begin work on the tile, any improvement until it is done (the passes are nearly free, and
-    // changes below eps would otherwise add up along a front: 640 x 384 1.41e-7 from FP64 at eps,
-    // 1.02e-7 so, the wave loop 1.20e-7).
-    float least = eps;
-    auto relax = [&](int k, float above, float below) -> bool {
+    // The update of cell k from its four neighbours.
+    auto update = [&](int k, float above, float below) -> float {
         // lanes 0 and 63 have no source lane and keep hx
         float l = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(hx[k]), __float_as_int(t[k]), 0x138, 0xF, 0xF, false));
         float r = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(hx[k]), __float_as_int(t[k]), 0x130, 0xF, 0xF, false));
         l = left ? hx[k] : l;
         r = right ? hx[k] : r;
         const float ax = umin_bits(l, r), ay = umin_bits(above, below);
-        const float n = godunov_raw(ax, ay, umin_bits(ax, ay), c[k]);
-        const bool imp = improves(n, t[k], least);
-        t[k] = umin_bits(t[k], n);
-        return imp;
+        return godunov_raw(ax, ay, umin_bits(ax, ay), c[k]);
     };
-    // One pass over the tile, rows down and (with several rows to a lane) up again.
-    auto pass = [&]() -> bool {
+    // The cells above and below this lane's.
+    auto ends = [&](float& first, float& last) {
         const float pu = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (L - TW), __float_as_int(t[R - 1])));
         const float pd = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (L + TW), __float_as_int(t[0])));
-        const float first = top ? ht : pu, last = bottom ? hb : pd;
+        first = top ? ht : pu;
+        last = bottom ? hb : pd;
+    };
+    // One pass over the tile, rows down and (with several rows to a lane) up again; whether a cell
+    // fell.  Work on a tile goes on until none does, whatever eps: the passes are nearly free, and
+    // changes below eps would otherwise add up along a front (640 x 384 1.41e-7 from FP64 at eps,
+    // 1.02e-7 so, the wave loop 1.20e-7).
+    auto pass = [&]() -> bool {
+        float first, last;
+        ends(first, last);
+        bool fell = false;
+        auto relax = [&](int k) {
+            const float n = update(k, k ? t[k - 1] : first, k + 1 < R ? t[k + 1] : last);
+            fell |= __float_as_uint(n) < __float_as_uint(t[k]);
+            t[k] = umin_bits(t[k], n);
+        };
+#pragma unroll
+        for (int k = 0; k < R; ++k) relax(k);
+#pragma unroll
+        for (int k = R - 2; k >= 0; --k) relax(k);
+        return __ballot(fell) != 0ull;
+    };
+    // Whether a cell would improve by eps, which begins work on the tile.  No time changes: an
+    // improvement below eps that was kept here would be published to no one, and the next one
+    // would be measured against it, so that many of them left the neighbours behind without limit.
+    auto unsettled = [&]() -> bool {
+        float first, last;
+        ends(first, last);
         bool imp = false;
 #pragma unroll
-        for (int k = 0; k < R; ++k) imp |= relax(k, k ? t[k - 1] : first, k + 1 < R ? t[k + 1] : last);
-#pragma unroll
-        for (int k = R - 2; k >= 0; --k) imp |= relax(k, k ? t[k - 1] : first, t[k + 1]);
+        for (int k = 0; k < R; ++k)
+            imp |= improves(update(k, k ? t[k - 1] : first, k + 1 < R ? t[k + 1] : last), t[k], eps);
         return __ballot(imp) != 0ull;
     };
     float nx[R], nt = inf, nb = inf;
@@ -279,7 +298,6 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
     for (;;) {
         if (work) {
             __builtin_amdgcn_s_setprio(kWorkPriority);
-            least = 0.0f;
             bool visible = (st & 1u) != 0u;         // (the first counter is odd from the start)
             if (!(st & 1u)) {
                 ++st;
@@ -305,7 +323,6 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
             }
             work = false;
             __builtin_amdgcn_s_setprio(0);
-            least = eps;
         }
         if (st & 1u) {
             wait_stores();
@@ -317,7 +334,7 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
             look();
             cmd = __builtin_amdgcn_readfirstlane(ld_agent(&a.cmd[rank]));
             if (take()) {
-                work = pass();
+                work = unsettled();
                 if (work) break;
             } else if (cmd == kCmdDone || cmd == kCmdAbort) {
                 break;
