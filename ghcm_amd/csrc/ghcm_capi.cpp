@@ -765,7 +765,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                          o_want = part(owned > 1 && !scan ? 4ull * kResMaxGroups * ra.want_stride : 0),
                          o_tile = part(sizeof(ResTile) * (size_t)T), o_state = part(8ull * states),
                          o_report = part(8ull * states), o_cmd = part(4ull * states), o_ctl = part(4ull * kResCtlWords),
-                         o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
+                         o_seeds = part(source_bytes(n_seeds_total, T, tw * th));
             if (resident_room(need)) {
                 char* const base = ctx->resident.as<char>();
                 ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);
@@ -782,8 +782,8 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                 if ((rc = prof_events(&e0, &e1))) return rc;
                 const GhcmInst* const inst_view = ctx->h_inst.dev_as<GhcmInst>();
                 const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
-                HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, seeds_view, groups, kind, st)
-                                  : wk.init(ra, inst_view, seeds_view, kind, st));
+                HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, d_inst, seeds_view, groups, kind, st)
+                                  : wk.init(ra, inst_view, d_inst, seeds_view, kind, st));
                 HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
                 if ((rc = await_resident(ra.tag, e0, e1))) return rc;
             }
@@ -810,7 +810,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
             const size_t o_edges = part(4ull * kRes3Words * T),
                          o_tile = part(sizeof(ResTile3) * (size_t)T), o_state = part(8ull * kRes3MaxGroups),
                          o_report = part(8ull * kRes3MaxGroups), o_cmd = part(4ull * kRes3MaxGroups),
-                         o_ctl = part(4ull * kResCtlWords), o_seeds = part(16ull * std::max<uint64_t>(1, n_seeds_total));
+                         o_ctl = part(4ull * kResCtlWords), o_seeds = part(source_bytes(n_seeds_total, T, tw * th * td));
             if (resident_room(need)) {
                 char* const base = ctx->resident.as<char>();
                 ra.edges = reinterpret_cast<uint32_t*>(base + o_edges);

@@ -22,6 +22,13 @@ enum : uint32_t {
 constexpr uint32_t kResMaxGroups = 1024;     // work-groups whose states one of them watches
 constexpr uint32_t kResMaxScan = 16;         // tiles of one work-group that scans their borders
 constexpr uint32_t kResMaxOwned = 256;       // tiles of one work-group (one want a thread)
+// Up to this many sources every tile reads their list; with more it reads the marks of its own cells.
+constexpr uint32_t kResFewSources = 1024;
+__host__ __device__ constexpr bool many_sources(uint64_t n) { return n > kResFewSources; }
+// Bytes of the sources' part of the workspace, `cells` to a tile.
+constexpr size_t source_bytes(uint64_t n, uint64_t tiles, uint32_t cells) {
+    return many_sources(n) ? (size_t)(tiles * (cells / 8u + 4u)) : (size_t)(16u * n);
+}
 
 // What a work-group needs to open a tile: one read.
 struct alignas(16) ResTile {
@@ -41,7 +48,9 @@ struct alignas(16) ResTile {
 struct ResidentArgs {
     uint32_t        n_inst;
     ResTile*        rtile;   // [tiles] by rank (the order in which tiles are dealt out)
-    uint32_t*       seeds;   // [n_seeds] (x, y, instance, rank of its tile)
+    uint32_t*       seeds;   // few sources: [n_seeds] (x, y, instance, rank of its tile)
+                             // many: [tiles] by rank, a bit a cell, row by row, set where it is a source;
+                             // then [tiles] by rank, 1: holds a source
     uint32_t        n_seeds;
     uint32_t        tiles;
     float           eps;
@@ -64,9 +73,10 @@ struct ResidentKernel {
 };
 // Null launch where no resident form is built (64 x 64 sweep tiles only).
 ResidentKernel get_resident_kernel(int tile_w, int tile_h, int kind, int mode);
-// h_inst, h_seeds: device views of the mapped host instance table and source list.
-hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
-                                uint32_t groups, int kind, hipStream_t s);
+// h_inst, h_seeds: device views of the mapped host instance table and source list; d_inst: n_inst
+// records of device memory (written with many sources only).
+hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, GhcmInst* d_inst,
+                                const uint32_t* h_seeds, uint32_t groups, int kind, hipStream_t s);
 
 // The one-wave tiles (8x8, 16x16, 32x8, 32x32): one wave64 per tile, the tile in its registers.
 // Here `edges` holds the tiles' inboxes (`inbox_words` each: the cells across each border, written
@@ -74,7 +84,8 @@ hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, c
 constexpr uint32_t kResMaxWaveTiles = 8192;
 struct ResidentWaveKernel {
     hipError_t (*launch)(const ResidentArgs&, uint32_t groups, hipStream_t, hipEvent_t ev0, hipEvent_t ev1);
-    hipError_t (*init)(const ResidentArgs&, const GhcmInst* h_inst, const uint32_t* h_seeds, int kind, hipStream_t);
+    hipError_t (*init)(const ResidentArgs&, const GhcmInst* h_inst, GhcmInst* d_inst, const uint32_t* h_seeds, int kind,
+                       hipStream_t);
     int (*blocks_per_cu)();
     uint32_t inbox_words;
 };
@@ -97,7 +108,7 @@ struct alignas(16) ResTile3 {
 };
 struct Resident3Args {
     ResTile3*       rtile;   // [tiles] by rank
-    uint32_t*       seeds;   // [n_seeds]
+    uint32_t*       seeds;   // as in ResidentArgs, the cells plane by plane
     uint32_t        n_seeds, tiles;
     float           eps;
     uint32_t*       edges;

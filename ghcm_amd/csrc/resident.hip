@@ -153,13 +153,17 @@ void k_resident_sweep(ResidentArgs a) {
     }
 
     __syncthreads();
-    for (uint32_t i = tid; i < a.n_seeds; i += kSweepThreads) {
-        const uint32_t r = a.seeds[4 * i + 3];
-        if (r % N == b) {
-            const uint32_t k = r / N;
-            atomicOr(&s_seeded[k >> 5], 1u << (k & 31u));
-            if constexpr (OWN == kOwnScan) s_key[k] = 0u;
-            if constexpr (OWN == kOwnWant) st_agent(&want[k], 0u);
+    auto seeded = [&](uint32_t k) {
+        atomicOr(&s_seeded[k >> 5], 1u << (k & 31u));
+        if constexpr (OWN == kOwnScan) s_key[k] = 0u;
+        if constexpr (OWN == kOwnWant) st_agent(&want[k], 0u);
+    };
+    if (many_sources(a.n_seeds)) {
+        if ((uint32_t)tid < m && holds_source<TW * TH>(a, b + (uint32_t)tid * N)) seeded((uint32_t)tid);
+    } else {
+        for (uint32_t i = tid; i < a.n_seeds; i += kSweepThreads) {
+            const uint32_t r = a.seeds[4 * i + 3];
+            if (r % N == b) seeded(r / N);
         }
     }
     wait_stores();
@@ -262,7 +266,11 @@ void k_resident_sweep(ResidentArgs a) {
         const bool sources = fresh && ((s_seeded[k >> 5] >> (k & 31u)) & 1u);
         __syncthreads();
         if (fresh && tid == 0) s_opened[k >> 5] |= 1u << (k & 31u);
-        if (sources) {
+        if (sources && many_sources(a.n_seeds)) {
+#pragma unroll 1
+            for (int i = tid; i < TW * TH; i += kSweepThreads)
+                if (is_source<TW * TH>(a, b + k * N, (uint32_t)i)) t_s[(i / TW + 1) * PW + i % TW + 1] = 0.0f;
+        } else if (sources) {
             for (uint32_t i = tid; i < a.n_seeds; i += kSweepThreads) {
                 const int x = (int)(a.seeds[4 * i] - d.x0), y = (int)(a.seeds[4 * i + 1] - d.y0);
                 if (a.seeds[4 * i + 2] == d.inst && x >= 0 && x < sx && y >= 0 && y < sy) t_s[(y + 1) * PW + x + 1] = 0.0f;
@@ -664,9 +672,9 @@ ResidentKernel get_resident_kernel(int tw, int th, int kind, int mode) {
     return {nullptr, nullptr};
 }
 
-hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds,
-                                uint32_t groups, int kind, hipStream_t s) {
-    return launch_init<64, 64>(a, h_inst, h_seeds, groups, 256u, kResMaxGroups, kind, s);
+hipError_t launch_resident_init(const ResidentArgs& a, const GhcmInst* h_inst, GhcmInst* d_inst,
+                                const uint32_t* h_seeds, uint32_t groups, int kind, hipStream_t s) {
+    return launch_init<64, 64>(a, h_inst, d_inst, h_seeds, groups, 256u, kResMaxGroups, kind, s);
 }
 
 }  // namespace ghcm

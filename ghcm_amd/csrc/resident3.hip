@@ -127,7 +127,15 @@ void k_resident_sweep3(Resident3Args a) {
             c_s[s3_box(L + 1, w + 1, z + 1)] = L < sx && w < sy && z < sz ? cv[z] : inf;
     }
     bool seeded = false;
-    for (uint32_t i = tid; i < a.n_seeds; i += kS3Threads)
+    if (many_sources(a.n_seeds)) {
+        seeded = holds_source<kS3X * kS3Y * kS3Z>(a, b) != 0u;
+        if (seeded)
+#pragma unroll 1
+            for (int z = 0; z < kS3Z; ++z)
+                if (is_source<kS3X * kS3Y * kS3Z>(a, b, (uint32_t)((z * kS3Y + w) * kS3X + L)))
+                    t_s[s3_box(L + 1, w + 1, z + 1)] = 0.0f;
+    }
+    for (uint32_t i = tid; i < (many_sources(a.n_seeds) ? 0u : a.n_seeds); i += kS3Threads)
         if (a.seeds[4 * i + 3] == b) {
             t_s[s3_box((int)(a.seeds[4 * i] - d.x0) + 1, (int)(a.seeds[4 * i + 1] - d.y0) + 1,
                        (int)(a.seeds[4 * i + 2] - d.z0) + 1)] = 0.0f;
@@ -377,7 +385,8 @@ __global__ void k_resident3_init(Resident3Args a, const GhcmInst* h_inst, const 
     for (size_t i = i0; i < kResCtlWords; i += stride) a.ctl[i] = 0u;
     const GhcmInst in = h_inst[0];
     const uint32_t nx = in.tiles_x, ny = in.tiles_y, nz = in.tiles_z;
-    for (size_t i = i0; i < a.n_seeds; i += stride) {
+    if (many_sources(a.n_seeds)) clear_sources<kS3X * kS3Y * kS3Z>(a, i0, stride);
+    for (size_t i = i0; i < (many_sources(a.n_seeds) ? 0u : a.n_seeds); i += stride) {
         const uint32_t x = h_seeds[4 * i], y = h_seeds[4 * i + 1], z = h_seeds[4 * i + 2];
         a.seeds[4 * i] = x;
         a.seeds[4 * i + 1] = y;
@@ -407,6 +416,16 @@ __global__ void k_resident3_init(Resident3Args a, const GhcmInst* h_inst, const 
     }
 }
 
+// With many sources: each one's cell marked in its tile's bits (see k_resident_sources).
+__global__ void k_resident3_sources(Resident3Args a, const GhcmInst* h_inst, const uint32_t* h_seeds) {
+    const uint32_t nx = h_inst->tiles_x, ny = h_inst->tiles_y;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n_seeds; i += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t x = h_seeds[4 * i], y = h_seeds[4 * i + 1], z = h_seeds[4 * i + 2];
+        mark_source<kS3X * kS3Y * kS3Z>(a, rank3(nx, ny, x / kS3X, y / kS3Y, z / kS3Z),
+                                        (z % kS3Z * kS3Y + y % kS3Y) * kS3X + x % kS3X);
+    }
+}
+
 template <int KIND>
 static hipError_t launch_resident3_t(const Resident3Args& a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     if (a.tiles == 0 || a.tiles > kRes3MaxGroups) return hipErrorInvalidValue;
@@ -420,6 +439,8 @@ static hipError_t launch_resident3_t(const Resident3Args& a, hipStream_t s, hipE
 template <int KIND>
 static hipError_t launch_resident3_init_t(const Resident3Args& a, const GhcmInst* h_inst, const uint32_t* h_seeds, hipStream_t s) {
     hipLaunchKernelGGL((k_resident3_init<(int)field_bytes<KIND>()>), dim3(a.tiles), dim3(256), 0, s, a, h_inst, h_seeds);
+    if (many_sources(a.n_seeds))
+        hipLaunchKernelGGL(k_resident3_sources, sources_grid(a.n_seeds), dim3(256), 0, s, a, h_inst, h_seeds);
     return hipGetLastError();
 }
 

@@ -126,12 +126,34 @@ __device__ __forceinline__ void report_totals(const Args& a, unsigned long long 
     sys_store(&a.rec->totals_tag, a.tag);
 }
 
-// The state of a resident solve, in one launch: the tiles' records and the sources (with the
-// rank of their tile) from the mapped host tables, borders at +INF, every work-group busy.
-// N: work-groups the tiles are dealt out to; words: of a tile's borders; states: counters.
+// With many sources, a.seeds: whether cell `i` of the tile of this rank is one (row by row, of CELLS),
+// whether the tile holds one, and the marks made and cleared (by all threads of a grid).
+template <uint32_t CELLS, typename Args>
+__device__ __forceinline__ bool is_source(const Args& a, uint32_t rank, uint32_t i) {
+    return ((a.seeds[(size_t)rank * (CELLS / 32u) + (i >> 5)] >> (i & 31u)) & 1u) != 0u;
+}
+template <uint32_t CELLS, typename Args>
+__device__ __forceinline__ uint32_t& holds_source(const Args& a, uint32_t rank) {
+    return a.seeds[(size_t)a.tiles * (CELLS / 32u) + rank];
+}
+template <uint32_t CELLS, typename Args>
+__device__ __forceinline__ void mark_source(const Args& a, uint32_t rank, uint32_t i) {
+    atomicOr(&a.seeds[(size_t)rank * (CELLS / 32u) + (i >> 5)], 1u << (i & 31u));
+    holds_source<CELLS>(a, rank) = 1u;
+}
+template <uint32_t CELLS, typename Args>
+__device__ __forceinline__ void clear_sources(const Args& a, size_t i0, size_t stride) {
+    for (size_t i = i0; i < (size_t)a.tiles * (CELLS / 32u + 1u); i += stride) a.seeds[i] = 0u;
+}
+
+// The state of a resident solve, in one launch: the tiles' records and the sources (few: with the
+// rank of their tile; many: k_resident_sources follows) from the mapped host tables, borders at
+// +INF, every work-group busy.
+// N: work-groups the tiles are dealt out to; words: of a tile's borders; states: counters; d_inst:
+// with many sources, the instances for k_resident_sources.
 template <int TW, int TH, int FB>
-__global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const uint32_t* h_seeds, uint32_t N,
-                                uint32_t words, uint32_t states) {
+__global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, GhcmInst* d_inst, const uint32_t* h_seeds,
+                                uint32_t N, uint32_t words, uint32_t states) {
     const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     const uint4 inf4 = make_uint4(kInfBits, kInfBits, kInfBits, kInfBits);
     uint4* const e4 = reinterpret_cast<uint4*>(a.edges);
@@ -147,7 +169,11 @@ __global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const ui
         a.cmd[i] = 0u;
     }
     for (size_t i = i0; i < kResCtlWords; i += stride) a.ctl[i] = 0u;
-    for (size_t i = i0; i < a.n_seeds; i += stride) {
+    if (many_sources(a.n_seeds)) {
+        clear_sources<TW * TH>(a, i0, stride);
+        for (size_t j = i0; j < a.n_inst; j += stride) d_inst[j] = h_inst[j];
+    }
+    for (size_t i = i0; i < (many_sources(a.n_seeds) ? 0u : a.n_seeds); i += stride) {
         const uint32_t x = h_seeds[3 * i], y = h_seeds[3 * i + 1], j = h_seeds[3 * i + 2];
         const GhcmInst in = h_inst[j];
         a.seeds[4 * i] = x;
@@ -187,14 +213,32 @@ __global__ void k_resident_init(ResidentArgs a, const GhcmInst* h_inst, const ui
     }
 }
 
+// With many sources: each one's cell marked in its tile's bits, so that a tile reads only its own.
+// With every tile reading the whole list, 10^6 sources in 4096^2 took 7,980 us against 2,840 in the
+// wave loop and 512 in each of 200 fields 3,450 against 1,560; with marks 1,200 and 1,640.  The line
+// at kResFewSources (listed against marked): 1,024 sources in 256^2 81 and 84 us, in 1024^2 90 and 94,
+// in 512^2 of 8x8 tiles 82 and 82; 4,096 of them 89 and 86, 98 and 97, 87 and 72.
 template <int TW, int TH>
-static hipError_t launch_init(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds, uint32_t groups,
-                              uint32_t words, uint32_t states, int kind, hipStream_t s) {
+__global__ void k_resident_sources(ResidentArgs a, const GhcmInst* d_inst, const uint32_t* h_seeds) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n_seeds; i += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t x = h_seeds[3 * i], y = h_seeds[3 * i + 1], j = h_seeds[3 * i + 2];
+        mark_source<TW * TH>(a, resident_rank(d_inst[j], x / TW, y / TH), y % TH * TW + x % TW);
+    }
+}
+inline dim3 sources_grid(uint32_t n) { return dim3(n < 256u * 4096u ? (n + 255u) / 256u : 4096u); }
+
+template <int TW, int TH>
+static hipError_t launch_init(const ResidentArgs& a, const GhcmInst* h_inst, GhcmInst* d_inst, const uint32_t* h_seeds,
+                              uint32_t groups, uint32_t words, uint32_t states, int kind, hipStream_t s) {
     const dim3 grid(a.tiles < 1024u ? a.tiles : 1024u), block(256);
     if (kind <= 1)
-        hipLaunchKernelGGL((k_resident_init<TW, TH, 4>), grid, block, 0, s, a, h_inst, h_seeds, groups, words, states);
+        hipLaunchKernelGGL((k_resident_init<TW, TH, 4>), grid, block, 0, s, a, h_inst, d_inst, h_seeds, groups, words,
+                           states);
     else
-        hipLaunchKernelGGL((k_resident_init<TW, TH, 2>), grid, block, 0, s, a, h_inst, h_seeds, groups, words, states);
+        hipLaunchKernelGGL((k_resident_init<TW, TH, 2>), grid, block, 0, s, a, h_inst, d_inst, h_seeds, groups, words,
+                           states);
+    if (many_sources(a.n_seeds))
+        hipLaunchKernelGGL((k_resident_sources<TW, TH>), sources_grid(a.n_seeds), block, 0, s, a, d_inst, h_seeds);
     return hipGetLastError();
 }
 

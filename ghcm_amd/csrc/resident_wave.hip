@@ -184,8 +184,13 @@ __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
     uint32_t* const out_t = box(1) + x;
     uint32_t* const out_b = box(3) + x;
 
-    bool work = false;
-    for (uint32_t i0 = 0; i0 < a.n_seeds; i0 += 64) {
+    bool work = many_sources(a.n_seeds) && holds_source<TW * TH>(a, rank) != 0u;
+    if (work) {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (is_source<TW * TH>(a, rank, (uint32_t)((g * R + k) * TW + x))) t[k] = 0.0f;
+    }
+    for (uint32_t i0 = 0; i0 < (many_sources(a.n_seeds) ? 0u : a.n_seeds); i0 += 64) {
         const uint32_t i = min(i0 + (uint32_t)L, a.n_seeds - 1u);
         unsigned long long mine = __ballot(a.seeds[4 * i + 3] == rank);
         const uint32_t px = a.seeds[4 * i] - d.x0, py = a.seeds[4 * i + 1] - d.y0;
@@ -407,9 +412,9 @@ static int occ_wave_t() {
 }
 
 template <int TW, int TH>
-static hipError_t launch_wave_init_t(const ResidentArgs& a, const GhcmInst* h_inst, const uint32_t* h_seeds, int kind,
-                                     hipStream_t s) {
-    return launch_init<TW, TH>(a, h_inst, h_seeds, a.tiles, inbox_words<TW, TH>(), kResMaxWaveTiles, kind, s);
+static hipError_t launch_wave_init_t(const ResidentArgs& a, const GhcmInst* h_inst, GhcmInst* d_inst, const uint32_t* h_seeds,
+                                     int kind, hipStream_t s) {
+    return launch_init<TW, TH>(a, h_inst, d_inst, h_seeds, a.tiles, inbox_words<TW, TH>(), kResMaxWaveTiles, kind, s);
 }
 
 template <int TW, int TH>
