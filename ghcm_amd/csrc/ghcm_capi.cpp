@@ -688,7 +688,12 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // 4096^2 (four) 1,670 -> 950 us, a batch of 512 (143) 20.6 -> 10.3 ms.
     // Up to kResMaxScan tiles each, work-groups scan the borders of their closed tiles, above it
     // they are told: four tiles 1,040 against 1,130 us, eight 2,080 against 2,260, eleven 3,015
-    // against 3,300, 15 equal, a batch of 21 each 3,600 against 3,110.
+    // against 3,300, 15 equal, a batch of 21 each 3,600 against 3,110.  With many fronts at work most
+    // tiles are wanted at once and the scan of them all is what takes the time: from 64 sources the
+    // line lies at 6 tiles each (scanned against told, 100 sources: four tiles 526 and 553 us, six 820
+    // and 831, eight 979 and 957, 15 1,723 and 1,522; batches of one source to a field: four 590 and
+    // 600, seven 882 and 842, 16 1,611 and 1,431; 16 with 128 to a field 1,598 and 1,366, which the
+    // wave loop took 1,503 for).
     // The one-wave tiles (resident_wave.hip) likewise, one wave64 per tile with the tile in
     // registers, up to the resident waves (8,184 tiles of 8x8 or 6,136 of 16x16 on 256 CUs; larger
     // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
@@ -744,7 +749,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                                     : wk.launch && T <= kResMaxWaveTiles && groups + 1u <= fit;
         if (fits) {
             const uint32_t owned = rk.launch ? (T + groups - 1) / groups : 1u;
-            const bool scan = owned <= kResMaxScan;
+            const bool scan = owned <= (n_seeds_total < kResScanSources ? kResMaxScan : kResAlwaysScan);
             const uint32_t states = rk.launch ? kResMaxGroups : kResMaxWaveTiles;
             ResidentArgs ra{};
             ra.n_inst = n_inst;

@@ -20,7 +20,9 @@ enum : uint32_t {
 };
 
 constexpr uint32_t kResMaxGroups = 1024;     // work-groups whose states one of them watches
-constexpr uint32_t kResMaxScan = 16;         // tiles of one work-group that scans their borders
+constexpr uint32_t kResMaxScan = 16;         // tiles of one work-group that scans their borders,
+constexpr uint32_t kResAlwaysScan = 6;       // with this many sources or more, tiles up to which it does
+constexpr uint32_t kResScanSources = 64;
 constexpr uint32_t kResMaxOwned = 256;       // tiles of one work-group (one want a thread)
 // Up to this many sources every tile reads their list; with more it reads the marks of its own cells.
 constexpr uint32_t kResFewSources = 1024;

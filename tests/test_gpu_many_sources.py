@@ -68,6 +68,32 @@ def test_batch(rng, n_inst, each):
             t.free()
 
 
+# about eleven tiles to a work-group: borders scanned up to 63 sources in all, owners told from 64
+@pytest.mark.parametrize("n", [63, 64])
+def test_sources_where_the_scan_ends(rng, n):
+    costs = [rng.uniform(0.1, 10.0, (300, 300) if i % 40 else (500, 1100)).astype(np.float32) for i in range(440)]
+    total = [0] * 440
+    for k in range(n):
+        total[(k * 40) % 440 if k % 2 else k] += 1
+    seeds = [_sources(rng, c.shape, k)[:k] if k > 1 else np.array([(7, 290)] * k, np.uint32).reshape(-1, 2)
+             for c, k in zip(costs, total)]
+    assert sum(len(s) for s in seeds) == n
+    print(f"case {n} sources in 440 fields", flush=True)
+    with g.Context(0, **dict(SWEEP, n_active=65536)) as ctx:
+        dev = [(ctx.to_device(c), ctx.alloc(c.shape, np.float32)) for c in costs]
+        st = ctx.solve_batch(g.FIELD_COST_F32, [(d.ptr, t.ptr, c.shape[1], c.shape[0], s)
+                                                for (d, t), c, s in zip(dev, costs, seeds)])
+        assert st["converged"] == 1 and st["tiles_total"] > 10 * 1024
+        for (d, t), c, s in zip(dev, costs, seeds):
+            got = t.download()
+            if len(s):
+                check(got, oracle.fmm_f32(c, s), s, c, label=f"{c.shape}")
+            else:
+                assert np.all(np.isinf(got))
+            d.free()
+            t.free()
+
+
 @pytest.mark.parametrize("n", [1024, 1026, 20000, 13 * 41 * 70])
 def test_volume(rng, n):
     cost = (1.0 / rng.uniform(0.2, 5.0, (13, 41, 70))).astype(np.float32)
