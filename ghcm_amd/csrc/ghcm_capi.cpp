@@ -439,6 +439,32 @@ uint32_t noalloc_max_tiles(uint32_t edge_h) {
     return lo;
 }
 
+// Solves in flight on a device, of every context, that as resident solves take more than half of
+// its work-groups each (of one-wave tiles more than three quarters).  Two such alternate faster than
+// two wave loops run together; of three and more the waves fill each other's gaps, which resident
+// solves, each bound by latency, cannot: 3000^2 in 1, 2, 3 and 8 threads, waves 1,327, 801, 623 and
+// 564 us a solve, resident 777, 774, 818 and 766; 2048^2 829, 501, 372 and 328 against 396, 371, 372
+// and 371; a volume of 150 x 90 x 61 641, 348, 245 and 196 against 384, 352, 322 and 272; 700^2 in
+// 8x8 tiles 1,645, 845, 582 and 482 against 440, 655, 654 and 610.  Smaller ones run beside each other:
+// 1300^2 in 8 threads 177 against 126, 600^2 in 8x8 tiles 366 against 328.  So one that finds
+// kLargeTogether others goes by waves.
+constexpr uint32_t kLargeTogether = 2;
+class LargeSolve {
+public:
+    ~LargeSolve() {
+        if (n_) n_->fetch_sub(1, std::memory_order_relaxed);
+    }
+    // Counts the caller's solve; whether it may be a resident one.
+    bool enter(int ordinal) {
+        static std::atomic<uint32_t> in_flight[64];
+        n_ = &in_flight[(unsigned)ordinal % 64u];
+        return n_->fetch_add(1, std::memory_order_relaxed) < kLargeTogether;
+    }
+
+private:
+    std::atomic<uint32_t>* n_ = nullptr;
+};
+
 int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst, ghcm_stats* stats,
                     bool three_d, bool noalloc) {
     const auto t_wall0 = std::chrono::steady_clock::now();
@@ -699,6 +725,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
     // 16x16 FIM tiles 3,837 -> 455 us.
     bool resident_done = false;
+    LargeSolve large_solve;             // until the solve ends
     // The events that stamp a resident launch, when kernels are profiled.
     auto prof_events = [&](hipEvent_t* e0, hipEvent_t* e1) -> int {
         if (!cfg.profile_kernels) return GHCM_OK;
@@ -747,7 +774,8 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
         const uint32_t groups = rk.launch ? (uint32_t)std::min<uint64_t>({fit, kResMaxGroups, T}) : (T + 7u) / 8u;
         const bool fits = rk.launch ? groups && (uint64_t)T <= (uint64_t)groups * kResMaxOwned
                                     : wk.launch && T <= kResMaxWaveTiles && groups + 1u <= fit;
-        if (fits) {
+        const bool large = rk.launch ? 2ull * groups > fit : 4ull * groups > 3ull * fit;
+        if (fits && (!large || large_solve.enter(ctx->ordinal))) {
             const uint32_t owned = rk.launch ? (T + groups - 1) / groups : 1u;
             const bool scan = owned <= (n_seeds_total < kResScanSources ? kResMaxScan : kResAlwaysScan);
             const uint32_t states = rk.launch ? kResMaxGroups : kResMaxWaveTiles;
@@ -800,7 +828,8 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     if (sweep3 && n_inst == 1 && cfg.launch_mode == 0 && cfg.max_waves == 0 && n_sel >= cus) {
         const Resident3Kernel rk = get_resident3_kernel(kind);
         const uint64_t fit = (uint64_t)std::max(0, rk.launch ? rk.blocks_per_cu() : 0) * cus;
-        if (rk.launch && T <= std::min<uint64_t>(fit, kRes3MaxGroups)) {
+        const bool large = 2ull * T > fit;
+        if (rk.launch && T <= std::min<uint64_t>(fit, kRes3MaxGroups) && (!large || large_solve.enter(ctx->ordinal))) {
             Resident3Args ra{};
             ra.tiles = T;
             ra.eps = cfg.min_change;
