@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <vector>
@@ -34,6 +36,20 @@ int no_throw(F&& body) noexcept {
         return fail(GHCM_ERR_INVALID_ARG, "%s", e.what());
     }
 }
+// What this process has at work on a device: solves of every context, and servers with requests.
+struct DeviceLoad {
+    std::mutex mu;
+    uint32_t servers = 0, waves = 0, resident = 0;  // solves by waves, and resident ones
+    uint32_t share = 0;                             // of the chip that the resident ones take
+    uint64_t cells = 0;                             // theirs
+    std::chrono::steady_clock::time_point left{};   // when a server or a solve by waves last ended,
+    std::thread::id left_by;                        // and whose thread it was
+    void leave() {
+        left = std::chrono::steady_clock::now();
+        left_by = std::this_thread::get_id();
+    }
+};
+DeviceLoad& device_load(int ordinal);
 // Validation shared by contexts and servers.
 int check_config(const ghcm_config* c);
 

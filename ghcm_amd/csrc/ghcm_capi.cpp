@@ -44,6 +44,11 @@ using ghcm_capi::kind_bytes;
 using ghcm_capi::no_throw;
 using ghcm_capi::valid_kind;
 
+ghcm_capi::DeviceLoad& ghcm_capi::device_load(int ordinal) {
+    static DeviceLoad load[64];
+    return load[(unsigned)ordinal % 64u];
+}
+
 namespace {
 thread_local std::string g_last_error;
 // Seeds the allocation-free solve accepts (its pinned seed list is sized when a context is
@@ -439,30 +444,65 @@ uint32_t noalloc_max_tiles(uint32_t edge_h) {
     return lo;
 }
 
-// Solves in flight on a device, of every context, that as resident solves take more than half of
-// its work-groups each (of one-wave tiles more than three quarters).  Two such alternate faster than
-// two wave loops run together; of three and more the waves fill each other's gaps, which resident
-// solves, each bound by latency, cannot: 3000^2 in 1, 2, 3 and 8 threads, waves 1,327, 801, 623 and
-// 564 us a solve, resident 777, 774, 818 and 766; 2048^2 829, 501, 372 and 328 against 396, 371, 372
-// and 371; a volume of 150 x 90 x 61 641, 348, 245 and 196 against 384, 352, 322 and 272; 700^2 in
-// 8x8 tiles 1,645, 845, 582 and 482 against 440, 655, 654 and 610.  Smaller ones run beside each other:
-// 1300^2 in 8 threads 177 against 126, 600^2 in 8x8 tiles 366 against 328.  So one that finds
-// kLargeTogether others goes by waves.
-constexpr uint32_t kLargeTogether = 2;
-class LargeSolve {
+// This solve's share in its device's load, and whether it may be a resident one beside the others.
+// A resident solve holds its work-groups, and what other streams have behind it in its hardware
+// queue, until it ends; the launches of wave loops are shared out.  So it runs beside no server that
+// has requests, no wave loop, and of resident solves only beside those of about its size, all of
+// which the chip holds at once.  Resident at all times, against now (as by waves): 8 requests of 900^2
+// each time beside a thread that solves 4096^2 17 ms, 1.9; 256^2 beside 4096^2 1,664 us, 288; 700^2
+// in 8x8 tiles beside 1024^2 27 ms, 2.4; and of several large ones the wave loops fill each other's gaps:
+// 3000^2 in 8 threads 766 us a solve, 560, a volume of 150 x 90 x 61 272, 197.  Equal ones that fit
+// are the faster resident: 256^2 in 8 threads 24 us a solve, by waves 51.
+class SolveInFlight {
 public:
-    ~LargeSolve() {
-        if (n_) n_->fetch_sub(1, std::memory_order_relaxed);
+    explicit SolveInFlight(int ordinal) : load_(ghcm_capi::device_load(ordinal)) {}
+    ~SolveInFlight() {
+        std::lock_guard<std::mutex> lk(load_.mu);
+        leave();
     }
-    // Counts the caller's solve; whether it may be a resident one.
-    bool enter(int ordinal) {
-        static std::atomic<uint32_t> in_flight[64];
-        n_ = &in_flight[(unsigned)ordinal % 64u];
-        return n_->fetch_add(1, std::memory_order_relaxed) < kLargeTogether;
+    SolveInFlight(const SolveInFlight&) = delete;
+    SolveInFlight& operator=(const SolveInFlight&) = delete;
+    // groups of the fit that the chip holds; cells: in all.
+    bool reside(uint64_t groups, uint64_t fit, uint64_t cells) {
+        const uint32_t share = (uint32_t)((groups * kWhole + fit - 1) / fit);
+        std::lock_guard<std::mutex> lk(load_.mu);
+        const uint64_t n = load_.resident;
+        if (load_.servers || load_.waves || load_.share + share > kWhole) return false;
+        if (load_.left_by != std::this_thread::get_id() && std::chrono::steady_clock::now() - load_.left < kLinger)
+            return false;
+        if (n && (2 * cells * n < load_.cells || cells * n > 2 * load_.cells)) return false;
+        ++load_.resident;
+        load_.share += share_ = share;
+        load_.cells += cells_ = cells;
+        return true;
+    }
+    void by_waves() {
+        std::lock_guard<std::mutex> lk(load_.mu);
+        leave();
+        ++load_.waves;
+        waves_ = true;
     }
 
 private:
-    std::atomic<uint32_t>* n_ = nullptr;
+    static constexpr uint32_t kWhole = 1u << 16;
+    // Another thread that has just ended its solve by waves, or its server's last request, is taken
+    // to come again (256^2 beside 2048^2 without this 3,748 solves/s, with it 3,995, by waves 3,959).
+    static constexpr std::chrono::microseconds kLinger{500};
+    void leave() {
+        if (waves_) {
+            --load_.waves;
+            load_.leave();
+        }
+        if (!share_) return;
+        --load_.resident;
+        load_.share -= share_;
+        load_.cells -= cells_;
+        share_ = 0;
+    }
+    ghcm_capi::DeviceLoad& load_;
+    uint32_t share_ = 0;            // of the chip, while resident
+    uint64_t cells_ = 0;
+    bool waves_ = false;
 };
 
 int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst, ghcm_stats* stats,
@@ -547,6 +587,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     const uint32_t T = (uint32_t)tiles64;
 
     HIP_TRY(hipSetDevice(ctx->ordinal));
+    SolveInFlight in_flight(ctx->ordinal);
     hipStream_t st = ctx->stream;
     const uint32_t shard_cap = (T + kShards - 1) / kShards;
     // The sweep kernels stage their halo columns from edge columns kept for every tile
@@ -725,7 +766,6 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
     // 16x16 FIM tiles 3,837 -> 455 us.
     bool resident_done = false;
-    LargeSolve large_solve;             // until the solve ends
     // The events that stamp a resident launch, when kernels are profiled.
     auto prof_events = [&](hipEvent_t* e0, hipEvent_t* e1) -> int {
         if (!cfg.profile_kernels) return GHCM_OK;
@@ -774,8 +814,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
         const uint32_t groups = rk.launch ? (uint32_t)std::min<uint64_t>({fit, kResMaxGroups, T}) : (T + 7u) / 8u;
         const bool fits = rk.launch ? groups && (uint64_t)T <= (uint64_t)groups * kResMaxOwned
                                     : wk.launch && T <= kResMaxWaveTiles && groups + 1u <= fit;
-        const bool large = rk.launch ? 2ull * groups > fit : 4ull * groups > 3ull * fit;
-        if (fits && (!large || large_solve.enter(ctx->ordinal))) {
+        if (fits && in_flight.reside(rk.launch ? groups : groups + 1u, fit, cells)) {
             const uint32_t owned = rk.launch ? (T + groups - 1) / groups : 1u;
             const bool scan = owned <= (n_seeds_total < kResScanSources ? kResMaxScan : kResAlwaysScan);
             const uint32_t states = rk.launch ? kResMaxGroups : kResMaxWaveTiles;
@@ -828,8 +867,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     if (sweep3 && n_inst == 1 && cfg.launch_mode == 0 && cfg.max_waves == 0 && n_sel >= cus) {
         const Resident3Kernel rk = get_resident3_kernel(kind);
         const uint64_t fit = (uint64_t)std::max(0, rk.launch ? rk.blocks_per_cu() : 0) * cus;
-        const bool large = 2ull * T > fit;
-        if (rk.launch && T <= std::min<uint64_t>(fit, kRes3MaxGroups) && (!large || large_solve.enter(ctx->ordinal))) {
+        if (rk.launch && T <= std::min<uint64_t>(fit, kRes3MaxGroups) && in_flight.reside(T, fit, cells)) {
             Resident3Args ra{};
             ra.tiles = T;
             ra.eps = cfg.min_change;
@@ -863,7 +901,10 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
             }
         }
     }
-    if (!resident_done && (rc = enqueue_init())) return rc;
+    if (!resident_done) {
+        in_flight.by_waves();
+        if ((rc = enqueue_init())) return rc;
+    }
 
     // launch_mode 3: tile solve and wave boundary in one launch (sweep kernel).
     const SolveKernel fk = get_fused_kernel((int)tw, (int)th, kind, cfg.kernel);

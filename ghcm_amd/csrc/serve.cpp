@@ -523,6 +523,19 @@ int ghcm_server::loop() {
     uint32_t n_live = 0;
     uint64_t idle_spins = 0;
     char* base = arena.as<char>();
+    // The device's load shows this server while it has requests.
+    struct Busy {
+        ghcm_capi::DeviceLoad& load;
+        bool on;
+        ~Busy() { set(false); }
+        void set(bool b) {
+            if (b == on) return;
+            std::lock_guard<std::mutex> lk(load.mu);
+            if (b) ++load.servers; else --load.servers;
+            if (!b) load.leave();
+            on = b;
+        }
+    } busy{ghcm_capi::device_load(ordinal), false};
     for (;;) {
         bool progressed = false;
         std::vector<Request*> batch;
@@ -532,8 +545,10 @@ int ghcm_server::loop() {
                 if (stop && !drain) return GHCM_OK;
                 if (n_live > 0 || !finishing.empty() || !pending.empty()) break;
                 if (stop) return GHCM_OK;           // drained
+                busy.set(false);
                 cv_work.wait(lk);
             }
+            busy.set(true);
             while (!pending.empty() && place(pending.front())) {
                 batch.push_back(pending.front());
                 pending.pop_front();
