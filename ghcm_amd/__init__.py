@@ -152,7 +152,7 @@ EXPORTED_SYMBOLS = (
     "ghcm_field_load_mono", "ghcm_field_load_rgb_luminosity", "ghcm_rgb_luminosity_device",
     "ghcm_write_time_field_png", "ghcm_write_field_hdr", "ghcm_blob_write", "ghcm_blob_read",
     "ghcm_test_run", "ghcm_field_cost_sin_checkerboard", "ghcm_field_cost_random",
-    "ghcm_tile_info", "ghcm_debug_select", "ghcm_solve_device_noalloc",
+    "ghcm_tile_info", "ghcm_debug_select", "ghcm_debug_refuse_resident", "ghcm_solve_device_noalloc",
 )
 
 _lib = None
@@ -244,6 +244,7 @@ def lib() -> ctypes.CDLL:
     L.ghcm_tile_info.argtypes = [u32, u32, u32, u32, u32, u32, P(TileDesc)]
     L.ghcm_debug_select.argtypes = [vp, u32, vp, vp, vp, u32, u32, i32, vp, P(u32), vp, P(u32),
                                     vp, vp, vp, P(u32)]
+    L.ghcm_debug_refuse_resident.argtypes = [vp, i32]
     for name in EXPORTED_SYMBOLS:
         getattr(L, name).restype = getattr(L, name).restype or i32
     _lib = L
@@ -502,6 +503,10 @@ class Context:
                                          nmasks.ctypes.data, ctypes.byref(nn)))
         return (jobs[:nj.value], handed[:nh.value], nxt[:nn.value], nkeys[:nn.value],
                 nmasks[:nn.value])
+
+    def debug_refuse_resident(self, on: bool) -> None:
+        """Whether resident solves are given up as they start (test support)."""
+        _check(self._L.ghcm_debug_refuse_resident(self._h, 1 if on else 0))
 
 
 def tile_info(w: int, h: int, tile_w: int, tile_h: int, tile: int, tile_base: int = 0) -> dict:

@@ -89,6 +89,7 @@ struct ghcm_ctx {
     PinnedBuf h_ctrl, h_seeds, h_inst, h_jobs, h_status;
     PinnedBuf rec;                       // HostRec written by the wave loop
     uint32_t solve_seq = 0;              // tags the totals of each solve
+    bool refuse_resident = false;        // tests: resident solves are given up as they start
 };
 
 // ---------------------------------------------------------------------------------------
@@ -856,6 +857,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                 const uint32_t* const seeds_view = ctx->h_seeds.dev_as<uint32_t>();
                 HIP_TRY(rk.launch ? launch_resident_init(ra, inst_view, d_inst, seeds_view, groups, kind, st)
                                   : wk.init(ra, inst_view, d_inst, seeds_view, kind, st));
+                if (ctx->refuse_resident) HIP_TRY(launch_fill_u32(ra.ctl + kResDecision, 1, 2u, st));
                 HIP_TRY((rk.launch ? rk.launch : wk.launch)(ra, groups, st, e0, e1));
                 if ((rc = await_resident(ra.tag, e0, e1))) return rc;
             }
@@ -896,6 +898,7 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
                 hipEvent_t e0 = nullptr, e1 = nullptr;
                 if ((rc = prof_events(&e0, &e1))) return rc;
                 HIP_TRY(rk.init(ra, ctx->h_inst.dev_as<GhcmInst>(), ctx->h_seeds.dev_as<uint32_t>(), st));
+                if (ctx->refuse_resident) HIP_TRY(launch_fill_u32(ra.ctl + kResDecision, 1, 2u, st));
                 HIP_TRY(rk.launch(ra, st, e0, e1));
                 if ((rc = await_resident(ra.tag, e0, e1))) return rc;
             }
@@ -1509,6 +1512,12 @@ extern "C" int ghcm_tile_info(uint32_t w, uint32_t h, uint32_t tile_w, uint32_t 
         out->border_bit[s] = border_bit_across(s);
     }
     out->seed_tile = tile_of_cell(tile_base, tx_n, out->x0 + out->w - 1, out->y0 + out->h - 1, tile_w, tile_h);
+    return GHCM_OK;
+}
+
+extern "C" int ghcm_debug_refuse_resident(ghcm_ctx* ctx, int on) {
+    if (!ctx) return fail(GHCM_ERR_INVALID_ARG, "ctx is null");
+    ctx->refuse_resident = on != 0;
     return GHCM_OK;
 }
 

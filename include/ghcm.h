@@ -397,6 +397,10 @@ int ghcm_debug_select(ghcm_ctx* ctx, uint32_t tiles_total, const uint32_t* tiles
                       uint32_t* n_handed, uint32_t* next, float* next_keys,
                       uint32_t* next_masks, uint32_t* n_next);
 
+/* on != 0: the resident solves of this context find, when they start, that they have been given
+ * up for want of work-groups, and are solved by waves.  A test entry point. */
+int ghcm_debug_refuse_resident(ghcm_ctx* ctx, int on);
+
 #ifdef __cplusplus
 }
 #endif
