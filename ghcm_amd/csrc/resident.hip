@@ -378,6 +378,9 @@ void k_resident_sweep(ResidentArgs a) {
                 }
                 first = false;
                 ++rounds;
+                // The withdrawal is complete before the next look: a wave with a neighbour has waited
+                // for loads that it issued later.
+                if (OWN == kOwnWant && w == 0 && __ballot(act) == 0ull) wait_stores();
                 const bool stop = (rounds & 1023u) == 0u && must_stop(a.ctl, a.cmd, b, N, t_start);
                 uint32_t r = any4((__ballot(ch) ? 1u : 0u) | (__ballot(stop) ? 4u : 0u));
                 if (!(r & 1u)) {
@@ -507,13 +510,15 @@ void k_resident_sweep(ResidentArgs a) {
                 best = __builtin_amdgcn_readfirstlane(best);
                 bk = __builtin_amdgcn_readfirstlane(bk);
                 if (best != kInfBits) {
-                    // Each wave withdraws the want before it reads its side's border (open() waits
-                    // for the tile's record first): what is announced later is seen by the looks
-                    // at the open tile.
+                    // Each wave withdraws the want before it reads its side's border: open() waits
+                    // for the tile's record first, which it reads after the withdrawal (the barrier
+                    // to the compiler keeps it so, and vector memory completes in order).  What is
+                    // announced later is seen by the looks at the open tile.
                     if constexpr (OWN == kOwnScan) {
                         if (tid == 0) s_key[bk] = kInfBits;
                     } else {
                         if (L == 0) st_agent(&want[bk], kInfBits);
+                        __asm__ volatile("" ::: "memory");
                     }
                     // The visit counter turns odd before anything of the new tile is published.
                     if (!(st & 1u)) {
