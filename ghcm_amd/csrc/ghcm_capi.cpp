@@ -763,9 +763,9 @@ int solve_core_body(ghcm_ctx* ctx, int kind, const HostInst* hi, uint32_t n_inst
     // 600, seven 882 and 842, 16 1,611 and 1,431; 16 with 128 to a field 1,598 and 1,366, which the
     // wave loop took 1,503 for).
     // The one-wave tiles (resident_wave.hip) likewise, one wave64 per tile with the tile in
-    // registers, up to the resident waves (8,184 tiles of 8x8 or 6,136 of 16x16 on 256 CUs; larger
-    // grids keep the wave loop): 512^2 in 8x8 systolic tiles 4,595 -> 1,318 us, 640 x 384 in
-    // 16x16 FIM tiles 3,837 -> 455 us.
+    // registers, up to the resident waves (8,184 tiles of 8x8, 6,136 of 16x16 and 32x8 and 2,040 of
+    // 32x32 on 256 CUs; larger grids keep the wave loop): 512^2 in 8x8 systolic tiles 3,852 -> 1,169
+    // us, 640 x 384 in 16x16 FIM tiles 3,130 -> 359 us.
     bool resident_done = false;
     // The events that stamp a resident launch, when kernels are profiled.
     auto prof_events = [&](hipEvent_t* e0, hipEvent_t* e1) -> int {

@@ -1721,7 +1721,7 @@ __global__ void k_seed_serve(SolveArgs a, const uint32_t* seeds, uint32_t n_seed
 // and (tw != 0, sweep kernel) its tiles' edge columns initialised.  The loop leaves its idle state,
 // so that the next wave boundary reports the new slots, with or without seeds.  Bound by launches:
 // with one per request, 3-5 us each, the GPU waits 2-10 us for the next (64 requests of 128^2 to
-// 1536^2 handed in at once: 2.92 -> 2.80 ms to the last result).
+// 1536^2 handed in at once, timed in turn six times: 1.01 to 1.03 times as fast, 3,521 -> 3,458 us).
 template <int KIND>
 __global__ void k_admit_tiles(SolveArgs a, const AdmitRec* recs, uint32_t tw, uint32_t th) {
     const AdmitRec r = recs[blockIdx.y];
@@ -2306,7 +2306,7 @@ __device__ void sweep3_tile(const SolveArgs& a, uint32_t g, uint32_t wave, uint3
     for (;;) {
         // Wave w runs octant w: bit 0 -x, bit 1 -y, bit 2 -z (the branch is wave-uniform).
         // The sweeps, one chain of dependent steps, are issued before what the CU's other
-        // work-groups stage and commit: 256^3 3,565 -> 3,460 and 3,775 -> 3,704 us.  (Staging
+        // work-groups stage and commit: 256^3 1.03 to 1.04 times as fast in six runs in turn.  (Staging
         // first: no gain, and none of either in the 2-D sweep kernel.)
         __builtin_amdgcn_s_setprio(2);
         switch (w) {

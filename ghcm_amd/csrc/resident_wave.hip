@@ -12,12 +12,14 @@
 //              by the neighbour that owns the cell (agent-scope stores, published and read by the
 //              rules of resident.hip).  A look at all neighbours is one run of 128 bytes for an
 //              8x8 tile; its loads are in flight while kPasses passes run.
+//   work       a tile is worked on from a cell that would improve by eps until none falls at all;
+//              while it is idle none of its times changes.
 //   end        as in resident.hip, the counters per tile and watched by a work-group of its own.
 //
 // Bound by the round trip of a border through the memory side (about 1 us) per crossing.  Measured
-// (MI355X, whole calls, wave loop -> this): 512^2 rings in 8x8 systolic tiles 4,595 -> 1,318 us,
-// 640 x 384 smooth in 16x16 FIM tiles 3,837 -> 455, 700 x 500 smooth in 8x8 / 16x16 / 32x8
-// systolic and 32x32 FIM tiles 1,463 / 1,341 / 2,187 / 9,356 -> 465 / 452 / 489 / 960.
+// (MI355X, whole calls, wave loop -> this): 512^2 rings in 8x8 systolic tiles 3,852 -> 1,169 us,
+// 640 x 384 smooth in 16x16 FIM tiles 3,130 -> 359, 700 x 500 smooth in 8x8 / 16x16 / 32x8
+// systolic and 32x32 FIM tiles 1,505 / 1,480 / 1,888 / 11,058 -> 417 / 434 / 459 / 979.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -53,9 +55,9 @@ __host__ __device__ constexpr uint32_t inbox_side(int s) {
 template <int TW, int TH, int KIND>
 __device__ __forceinline__ void resident_wave(const ResidentArgs& a) {
     constexpr int R = lane_rows<TW, TH>();
-    // Passes between two looks, about one look's latency: for 8x8 tiles 2, 4, 6, 9 and 14 of them
-    // 1,531, 1,318, 1,340, 1,466 and 1,610 us (512^2 rings), for 16x16 1, 2, 3, 5 and 8 582, 455,
-    // 481, 521 and 621 us (640 x 384), for 32x32 1, 2, 3 and 4 1,050, 963, 1,062 and 1,136 us.
+    // Passes between two looks, about one look's latency: for 8x8 tiles 2, 4, 6 and 9 of them 1,346,
+    // 1,169, 1,182 and 1,246 us (512^2 rings), for 16x16 1, 2, 3 and 5 443, 358, 369 and 398 us (640 x
+    // 384), for 32x32 1,034, 979, 1,112 and 1,360 us (700 x 500), 2,550, 2,700, 3,002 and 3,350 (1300^2).
     constexpr int kPasses = R == 1 ? 4 : 2;
     __shared__ uint32_t s_word;
     const int tid = threadIdx.x, L = tid & 63;
@@ -381,7 +383,8 @@ __global__ __launch_bounds__(kWaveGroup) void k_resident_wave(ResidentArgs a) {
 // are the trap handler's, so 80 let eight waves run on it and the 88 that the compiler takes by
 // itself only seven -- three of these work-groups per CU instead of four, which the occupancy query
 // does not know: grids of 6,137 to 8,184 tiles joined too few and went to the wave loop (640^2 to
-// 744 x 704: 2,770-3,390 us; now 700-850).  The larger tiles' vector registers allow six at most.
+// 744 x 704: 2,770-3,390 us; now 700-850).  Of 16x16 and
+// 32x8 tiles the vector registers (79) allow six, of 32x32 (212 to 228) two: 6,136 and 2,040 tiles.
 template <int KIND>
 __global__ __launch_bounds__(kWaveGroup) __attribute__((amdgpu_num_sgpr(80))) void k_resident_wave8(ResidentArgs a) {
     resident_wave<8, 8, KIND>(a);

@@ -87,19 +87,18 @@ typedef struct ghcm_config {
     int32_t  cache_mode;            /* ghcm_cache_mode (no effect, see above)         */
     int32_t  kernel;                /* ghcm_kernel                                    */
     int32_t  scheduler;             /* ghcm_scheduler                                 */
-    uint32_t inner_iter_cap;        /* in-tile passes per visit, 0 = until converged  */
+    uint32_t inner_iter_cap;        /* in-tile passes per visit, 0 = until converged
+                                       (no effect on a resident solve, see launch_mode) */
     uint32_t max_waves;             /* safety cap on waves, 0 = automatic             */
     uint32_t waves_per_poll;        /* device scheduler: waves kept enqueued ahead of
                                        the last executed wave boundary (at least 2),
-                                       0 = 4                                          */
+                                       0 = 4 (no effect on a resident solve)          */
     uint32_t profile_kernels;       /* 1: time every tile-solve launch with HIP events
-                                       (fills solve_kernel_us / solve_launches)       */
+                                       (fills solve_kernel_us / solve_launches, which is
+                                       1 for a resident solve)                        */
     uint32_t launch_mode;           /* device scheduler: 0 = one tile-solve launch per
-                                       wave (default; 64x64 sweep tiles, and grids of up to
-                                       8,184 systolic or FIM tiles, with n of at least one
-                                       tile per CU and no wave cap are solved by one
-                                       resident launch instead, without waves; so are
-                                       volumes of up to 512 sweep tiles),
+                                       wave (default), or, see below, one resident launch
+                                       without waves,
                                        1 = one persistent cooperative launch runs every
                                        wave where built (sweep kernel; its grid barrier
                                        pays agent-scope fences),
@@ -118,6 +117,19 @@ typedef struct ghcm_config {
                                        shapes run as 0); the allocation-free entry point
                                        takes 0 and 4 only                               */
 } ghcm_config;
+/* Resident solves.  With launch_mode 0, the device scheduler, n of at least one tile per CU and
+ * max_waves 0, one launch solves (on 256 CUs, all instances of a batch together)
+ *   64x64 sweep tiles            up to 262,144 (256 to a work-group),
+ *   8x8 systolic or FIM tiles    up to 8,184,
+ *   16x16 and 32x8               up to 6,136,
+ *   32x32                        up to 2,040,
+ *   volumes of 64x8x8 sweep tiles  up to 512;
+ * other shapes, more tiles and the allocation-free entry point go by waves.  So does a solve that
+ * finds, in this process and on its device, a server with requests, a solve by waves or a resident
+ * solve of another size or without room for it, and one whose work-groups are not all running
+ * within 200 us (other work on the device).  A resident solve is not interrupted: work that reaches
+ * the device while it runs waits for its end.  max_waves, set to any large number, keeps the wave
+ * loop. */
 
 /* Solve statistics (EikonalResult durations, src/eikonal.h:31-36, plus counters). */
 typedef struct ghcm_stats {
@@ -210,9 +222,9 @@ int ghcm_solve_device_noalloc(ghcm_ctx* ctx, const void* d_field, int field_kind
  * n_seeds (x, y, z) triples (host memory).  kernel GHCM_KERNEL_SWEEP solves 64x8x8
  * tiles with the eight octant sweeps (inner_iter_cap counts rounds of all eight), the
  * other kernels 8x8x8 tiles with in-tile passes; the device scheduler runs the wave loop,
- * or the one resident launch of launch_mode 0:
- * n_active, min_change, inner_iter_cap, waves_per_poll, max_waves and launch_mode 2
- * (graph replay) apply, the tile shape fields do not (stats report tile_w/h/d), and
+ * or one resident launch (see ghcm_config):
+ * n_active, min_change, max_waves and launch_mode 2 (graph replay) apply, and by waves
+ * inner_iter_cap and waves_per_poll; the tile shape fields do not (stats report tile_w/h/d), and
  * the host scheduler returns GHCM_ERR_UNSUPPORTED.  Host-buffer and device-buffer forms
  * as for the 2-D solve. */
 int ghcm_solve3d(ghcm_ctx* ctx, const void* field, int field_kind, uint32_t w, uint32_t h,
