@@ -42,12 +42,9 @@ struct DeviceLoad {
     uint32_t servers = 0, waves = 0, resident = 0;  // solves by waves, and resident ones
     uint32_t share = 0;                             // of the chip that the resident ones take
     uint64_t cells = 0;                             // theirs
-    std::chrono::steady_clock::time_point left{};   // when a server or a solve by waves last ended,
-    std::thread::id left_by;                        // and whose thread it was
-    void leave() {
-        left = std::chrono::steady_clock::now();
-        left_by = std::this_thread::get_id();
-    }
+    std::chrono::steady_clock::time_point served{};  // when a server's last request ended,
+    std::chrono::steady_clock::time_point left{};    // a solve by waves, and whose thread's it was
+    std::thread::id left_by;
 };
 DeviceLoad& device_load(int ordinal);
 // Validation shared by contexts and servers.

@@ -532,7 +532,7 @@ int ghcm_server::loop() {
             if (b == on) return;
             std::lock_guard<std::mutex> lk(load.mu);
             if (b) ++load.servers; else --load.servers;
-            if (!b) load.leave();
+            if (!b) load.served = Clock::now();
             on = b;
         }
     } busy{ghcm_capi::device_load(ordinal), false};

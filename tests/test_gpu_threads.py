@@ -66,8 +66,9 @@ def test_threads_no_slower_than_by_waves(n):
     assert here <= 8 / 7 * waves
 
 
-def _beside(call, seconds, **cfg):
-    """Median seconds of call() while a thread solves 4096^2 again and again."""
+def _beside(call, seconds, pause=0.0, **cfg):
+    """Seconds of call() while a thread solves 4096^2 again and again: the median of them, or with
+    pauses the 90th percentile."""
     side = 4096
     cost = np.ones((side, side), np.float32)
     stop = threading.Event()
@@ -88,6 +89,8 @@ def _beside(call, seconds, **cfg):
         try:
             until = time.perf_counter() + seconds
             while time.perf_counter() < until:
+                if pause:
+                    time.sleep(pause)
                 t0 = time.perf_counter()
                 call()
                 took.append(time.perf_counter() - t0)
@@ -97,14 +100,14 @@ def _beside(call, seconds, **cfg):
         d.free()
         t.free()
     assert not errs, errs
-    return float(np.median(took))
+    return float(np.quantile(took, 0.9 if pause else 0.5))
 
 
-@pytest.mark.parametrize("caller", ["solve", "server"])
+@pytest.mark.parametrize("caller", ["solve", "server", "sparse server"])
 def test_no_caller_waits_for_a_resident_solve(caller):
     """A small solve, or a server's requests, beside a thread of large solves: no longer than where
     that thread goes by waves (max_waves set).  Half as long again is allowed; waiting for resident
-    solves they took 5.8 and 9 times as long."""
+    solves they took 5.8 and 9 times as long, and with pauses of 2 ms 2.4 times."""
     cost = g.cost_from_speed(g.gen_smooth_speed(256, 256, 2, 16.0, 0.2, 5.0))
     ref = oracle.fmm_f32(cost, [(3, 3)])
     print(f"case {caller} beside 4096^2", flush=True)
@@ -116,12 +119,13 @@ def test_no_caller_waits_for_a_resident_solve(caller):
             here, waves = _beside(call, 0.5), _beside(call, 0.5, max_waves=1_000_000)
             out[0] = t.download()
     else:
+        pause = 0.002 if caller == "sparse server" else 0.0
         with g.Server(0, **dict(SWEEP, n_active=65536)) as srv:
             def call():
-                tickets = [srv.submit(cost, [(3, 3)]) for _ in range(4)]
+                tickets = [srv.submit(cost, [(3, 3)]) for _ in range(1 if pause else 4)]
                 for k, ticket in enumerate(tickets):
                     out[k] = srv.wait(ticket, 60.0)[0]
-            here, waves = _beside(call, 0.5), _beside(call, 0.5, max_waves=1_000_000)
+            here, waves = _beside(call, 0.5, pause), _beside(call, 0.5, pause, max_waves=1_000_000)
     print(f"  {1e6 * here:.0f} us, by waves {1e6 * waves:.0f}", flush=True)
     for t in out.values():
         check(t, ref, [(3, 3)], cost, label=caller)
