@@ -125,11 +125,11 @@ typedef struct ghcm_config {
  *   32x32                        up to 2,040,
  *   volumes of 64x8x8 sweep tiles  up to 512;
  * other shapes, more tiles and the allocation-free entry point go by waves.  So does a solve that
- * finds, in this process and on its device, a server with requests, a solve by waves or a resident
- * solve of another size or without room for it, and one whose work-groups are not all running
- * within 200 us (other work on the device).  A resident solve is not interrupted: work that reaches
- * the device while it runs waits for its end.  max_waves, set to any large number, keeps the wave
- * loop. */
+ * finds, in this process and on its device, a server that has requests (or had one in the last
+ * 10 ms), a solve by waves, or resident solves of another size or without room for it, and one
+ * whose work-groups are not all running within 200 us (other work on the device).  A resident
+ * solve is not interrupted: work that reaches the device while it runs waits for its end.
+ * max_waves, set to any large number, keeps the wave loop. */
 
 /* Solve statistics (EikonalResult durations, src/eikonal.h:31-36, plus counters). */
 typedef struct ghcm_stats {
